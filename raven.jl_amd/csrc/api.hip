@@ -79,6 +79,7 @@ struct rv_handle {
     int64_t *explicit_idx = nullptr;
     double *affine = nullptr, *vgeo = nullptr, *mji = nullptr, *sgeo = nullptr;
     double *Dt = nullptr, *Dw = nullptr, *winv = nullptr;
+    char *fdtab = nullptr;       // flux differencing: pair weights in the state type
     double *MJ = nullptr;
     double *cellJ = nullptr;     // brick handles: per-cell J that MJ is filled from
     double *partials = nullptr;  // reduction scratch
@@ -207,7 +208,7 @@ void free_handle(rv_handle *h)
                     h->partials, h->qtmp,       h->dtoc,     h->ctod_ptr, h->ctod_rows,
                     h->m_cells, h->m_partner,   h->m_kind,   h->m_sgeo,   h->m_halves,
                     h->m_delta, h->m_slot, h->cellJ,  h->relax_partials, h->eprod,
-                    h->relax_sums, h->m_pairs, h->vgeo32, h->mji32, h->sgeo32, h->mj32};
+                    h->relax_sums, h->m_pairs, h->fdtab, h->vgeo32, h->mji32, h->sgeo32, h->mj32};
     for (void *b : bufs)
         if (b)
             (void)hipFree(b);
@@ -619,6 +620,21 @@ int finish_setup(rv_handle *h, const double *D, const double *w)
         (rc = dalloc(h, &h->partials, (size_t)2 * RED_BLOCKS * h->ns)) ||
         (rc = refresh_geo32(h)))
         return rc;
+    if (h->vflux) {
+        // weights of the flux-differencing pairs (StageParams::fdtab)
+        std::vector<double> t64(2 * nq * nq);
+        for (int i = 0; i < nq; ++i)
+            for (int n = 0; n < nq; ++n) {
+                t64[i * nq + n] = Dw[i * nq + n] - D[i + nq * n];
+                t64[nq * nq + i * nq + n] = D[i + nq * n];
+            }
+        std::vector<float> t32(t64.begin(), t64.end());
+        const size_t bytes = t64.size() * (h->dtype == RV_F64 ? 8 : 4);
+        const char *src = h->dtype == RV_F64 ? reinterpret_cast<const char *>(t64.data())
+                                             : reinterpret_cast<const char *>(t32.data());
+        if ((rc = upload(h, &h->fdtab, src, bytes)))
+            return rc;
+    }
     KernelKey key{h->dim, nq, h->law, h->dtype == RV_F64 ? 8 : 4, h->geo, h->flux};
     key.vflux = h->vflux;
     h->launcher = find_stage_launcher(key);
@@ -879,6 +895,7 @@ StageParams stage_params(rv_handle *h)
     P.Dt = as_global(h->Dt);
     P.Dw = as_global(h->Dw);
     P.winv = as_global(h->winv);
+    P.fdtab = as_global(h->fdtab);
     P.gamma = h->gamma;
     for (int c = 0; c < 3; ++c)
         P.u[c] = h->u[c];
@@ -998,8 +1015,7 @@ int64_t relax_partials_count(const rv_handle *h)
 {
     if (h->vflux == 0)
         return plane3_relax_slots(h->nq, h->K, h->wpb);
-    const int cpb = fd_cells_per_workgroup((int)h->Np);
-    return (h->K + cpb - 1) / cpb;
+    return fd_workgroups(h->dim, h->nq, h->law, h->dtype == RV_F64 ? 8 : 4, h->vflux, h->K);
 }
 
 // ... and the most it can write whatever the waves per workgroup (the stride

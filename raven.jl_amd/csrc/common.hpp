@@ -74,6 +74,9 @@ struct StageParams {
     const double RV_GLOBAL *Dt;    // [i*Nq + n] = D[n,i]            (general)
     const double RV_GLOBAL *Dw;    // [i*Nq + n] = D[n,i] w_n / w_i  (affine)
     const double RV_GLOBAL *winv;  // [i] = 1/w_i
+    // flux differencing, in the state's type: [i*Nq + n] = D[n,i] w_n / w_i - D[i,n]
+    // (affine), then [i*Nq + n] = D[i,n] (general)
+    const void RV_GLOBAL *fdtab;
     double gamma;
     double u[3];
     // relaxation stage (the flux-differencing kernels built for it): dq = a dq + k
@@ -146,9 +149,54 @@ struct MortarParams {
 using MortarLauncher = int (*)(const MortarParams &, void *stream, int phase);
 MortarLauncher find_mortar_launcher(int dim, int nq, int law, int real_bytes, int flux);
 
-// Flux-differencing kernels (fluxdiff.hip): whole cells per workgroup, a
-// thread per node, at least 256 threads where a cell has fewer nodes
-constexpr int fd_cells_per_workgroup(int nodes) { return nodes >= 256 ? 1 : 256 / nodes; }
+// Flux-differencing kernels (fluxdiff.hip): whole cells per workgroup.  The
+// line kernel (2-D and 3-D): a lane per line of a cell (dim Nq^(dim-1) lines
+// each); 2-D fills one wave, 3-D takes few cells that leave few idle lanes in
+// 2 to 4 waves (Nq = 2 to 8: 192/192, 189/192, 192/192, 225/256, 108/128,
+// 147/192, 192/192 lanes; at Nq = 5, 5 cells in 6 waves leave 9 lanes idle
+// but took 110 us against 83 us per FP64 stage of 24^3 cells: two such
+// workgroups fit a CU and wait together).
+constexpr int fd_cells_per_workgroup(int dim, int nq)
+{
+    return dim == 2 ? 32 / nq : nq == 2 ? 16 : nq == 3 ? 7 : nq == 4 ? 4 : nq == 5 ? 3 : 1;
+}
+// The node kernel: a lane per node, in 1-D one wave, else up to 256 lanes or
+// one cell.
+constexpr int fd_node_cells(int dim, int nq)
+{
+    int np = 1;
+    for (int d = 0; d < dim; ++d)
+        np *= nq;
+    const int most = dim == 1 ? 64 : 256;
+    return np >= most ? 1 : most / np;
+}
+constexpr bool fd_has_line_kernel(int dim, int law, int vflux)
+{
+    return dim > 1 && law == LAW_EULER && vflux == FLUX_EC;
+}
+// Whether a launch over K cells takes the line kernel: from about one wave per
+// SIMD of the device on (FP64; FP32, whose chains are shorter, from 1.75).
+// Below, the chain of one wave and the fetch of its code are all that counts
+// (the line kernel's unrolled pairs are about 15 KB a wave); above, the line
+// kernel's half as many fluxes do.  Measured, us per Euler stage, line / node
+// (waves of the line kernel): 2-D Nq = 8 FP64, 40^2 cells (400) 20.5 / 12.5,
+// 100^2 (2500) 25.1 / 41.5; 3-D Nq = 6 FP64, 8^3 (1024) 24.6 / 21.3, 10^3
+// (2000) 26.5 / 33.1; 3-D Nq = 8, 8^3 (1536) FP64 39.0 / 48.9, FP32 23.0 /
+// 20.7; 24^3 FP64 315 / 658, FP32 185 / 260.
+inline bool fd_by_line(int dim, int nq, int law, int real_bytes, int vflux, int64_t K)
+{
+    if (!fd_has_line_kernel(dim, law, vflux))
+        return false;
+    const int c = fd_cells_per_workgroup(dim, nq);
+    const int waves = (c * dim * (dim == 2 ? nq : nq * nq) + 63) / 64;
+    return (K + c - 1) / c * waves >= (real_bytes == 8 ? 1152 : 1792);
+}
+inline int64_t fd_workgroups(int dim, int nq, int law, int real_bytes, int vflux, int64_t K)
+{
+    const int c = fd_by_line(dim, nq, law, real_bytes, vflux, K) ? fd_cells_per_workgroup(dim, nq)
+                                                                 : fd_node_cells(dim, nq);
+    return (K + c - 1) / c;
+}
 
 // Entropy passes of the relaxation LSRK step (entropy.hip).  Each pass runs
 // RELAX_BLOCKS workgroups over contiguous node ranges and leaves per workgroup

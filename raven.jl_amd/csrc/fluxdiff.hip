@@ -11,12 +11,35 @@
 // (surfaceflux, numericalfluxes.jl:27-37), the pairing of Raven's
 // entropy-conservation tests.
 //
-// The form is compute-bound (Nq (Nq - 1) / 2 two-point fluxes per line and
-// direction, two logarithms each for the entropy-conservative flux).  Whole
-// cells fill a workgroup with their states staged in LDS; each symmetric pair
-// is evaluated once by threads packed over the workgroup's pairs, and a thread
-// per node gathers the pair terms.  Affine cells evaluate only the row dir of
-// the two-point flux (their l_g has no other component).
+// Two kernels, chosen by fd_by_line (common.hpp):
+//
+// The line kernel (fd_stage; Euler with the entropy-conservative flux, grids
+// that fill the device): a lane owns a LINE (Nq nodes along one direction) of
+// a cell, and a workgroup the dim Nq^(dim-1) lines of each of its C cells.
+//  * phase 0: the workgroup reads its cells' states and leaves each node's
+//    primitives in LDS;
+//  * phase 1: each lane walks the Nq (Nq - 1) / 2 symmetric pairs of its line,
+//    every two-point flux evaluated once and added to both ends in registers,
+//    then adds the numerical fluxes of the two faces its line ends on (the
+//    line's index is the face node's);
+//  * phase 2: the directions' sums meet in LDS, in the primitives' place, one
+//    direction after another (fixed order, deterministic);
+//  * phase 3: the update, with lane-contiguous accesses; q comes from the
+//    caches a second time.
+// Affine cells read the velocities with the line's direction first (LDS holds
+// u, v, w, u, v), so that one code serves every direction and only row 0 of
+// the flux is formed; curved cells form the flux along the pair's metric
+// vector D[n,i] l_n - D[i,n] l_i.
+//
+// It is bound by FP64 (or unpacked FP32) vector issue and HBM together: 52 or
+// 60 instructions a pair (short or long series), 10.5 pairs a node at Nq = 8.
+// On 32^3 cells of Nq = 8 a stage takes 0.80 ms in FP64 (a thread per node
+// with the pairs' terms exchanged through an LDS buffer took 2.00 ms):
+// 2.95 GB moved (3.7 TB/s), vector units busy 61 % of the cycles.
+//
+// The node kernel (fd_stage_node; everything else): a lane per node, each pair
+// evaluated from both ends.  The fluxes of the central forms cost little, and
+// small grids wait for the chain of one wave.
 //
 // A relaxation stage (RX, the RLSRK step of odesolvers.jl:117-151) keeps
 // k = L(q) apart from a dq, forms dq = a dq + k at the end and leaves each
@@ -25,6 +48,8 @@
 //
 // Compiled once per (dim, precision) with -DFD_DIM and -DFD_REAL; api.hip asks
 // every unit for a launcher.
+#include <type_traits>
+
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -39,120 +64,218 @@ namespace rv {
 
 namespace {
 
-template <int DIM, int NS, int LAW, int VF, typename R>
+// F = atanh(f) / f = log(zeta) / 2f as a series in u = f^2, and 1 / 2F, the
+// factors of the logarithmic mean (a + b) / 2F (logavg, numericalfluxes.jl:
+// 9-22, zeta = a / b, f = (a - b) / (a + b)).  Two lengths: for u < LIMIT[k]
+// the TERMS[k] terms leave a remainder below the type's rounding (FP64:
+// u^8 / 17 < 6e-18 below 1e-2, u^4 / 9 < 1.2e-17 below 1e-4; FP32: u^4 / 9
+// and u^2 / 5 < 2e-9).
+template <typename R>
+struct LogSeries {
+    static constexpr int TERMS[2] = {sizeof(R) == 8 ? 8 : 4, sizeof(R) == 8 ? 4 : 2};
+    static constexpr double LIMIT[2] = {1e-2, 1e-4};
+    double f[8], g[8];
+    constexpr LogSeries() : f{}, g{}
+    {
+        for (int k = 0; k < 8; ++k)
+            f[k] = 1.0 / (2 * k + 1);
+        // the reciprocal series: sum_{j <= k} f_j g_{k-j} = 0 for k > 0
+        for (int k = 0; k < 8; ++k) {
+            double v = k == 0 ? 0.5 : 0.0;
+            for (int j = 1; j <= k; ++j)
+                v -= f[j] * g[k - j];
+            g[k] = v;
+        }
+    }
+};
+
+template <typename R, int SHORT>
+__device__ __forceinline__ R series_f(R u)
+{
+    constexpr LogSeries<R> c;
+    R v = R(c.f[c.TERMS[SHORT] - 1]);
+#pragma unroll
+    for (int k = c.TERMS[SHORT] - 2; k >= 0; --k)
+        v = v * u + R(c.f[k]);
+    return v;
+}
+template <typename R, int SHORT>
+__device__ __forceinline__ R series_g(R u)
+{
+    constexpr LogSeries<R> c;
+    R v = R(c.g[c.TERMS[SHORT] - 1]);
+#pragma unroll
+    for (int k = c.TERMS[SHORT] - 2; k >= 0; --k)
+        v = v * u + R(c.g[k]);
+    return v;
+}
+
+// 1 / x from the hardware estimate by Newton's method (x normal): two steps
+// from v_rcp_f64's about 2^-24, one from v_rcp_f32's 1 ulp
+__device__ __forceinline__ double recip(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ float recip(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+
+// A node of a line, what the two-point flux takes from it, and the flux of a
+// pair along a metric vector m (GEN) or along component 0 of the (permuted)
+// velocity.  LDS holds NC values per node: lds_values(q) writes the first
+// 2 + DIM (1 for advection).
+template <int DIM, int LAW, int VF, typename R, bool GEN>
 struct TwoPoint {
-    // row `row` of the dim x Ns two-point flux matrix between q1 and q2
-    __device__ static inline void rows(const Law<DIM, LAW, R> &law, const R *q1, const R *q2,
-                                       int row0, int nrows, R (*F)[NS])
-    {
-        if constexpr (VF == FLUX_CENTRAL || LAW == LAW_ADVECTION) {
-            for (int r = 0; r < nrows; ++r) {
-                R f1[NS], f2[NS];
-                law.flux_row(row0 + r, q1, f1);
-                law.flux_row(row0 + r, q2, f2);
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    F[r][s] = (f1[s] + f2[s]) / R(2);
-            }
-        } else {
-            ec_rows(law, q1, prim(law, q1), q2, prim(law, q2), row0, nrows, F);
-        }
-    }
+    static constexpr int NS = LawInfo<DIM, LAW>::NS;
+    static constexpr bool ADV = LAW == LAW_ADVECTION;
+    static constexpr bool EC = VF == FLUX_EC && !ADV;
+    static constexpr int NV = ADV ? 1 : 2 + DIM;
 
-    // Per-node quantities of the entropy-conservative flux: velocity u = rho u / rho,
-    // b = rho / 2p with p = (gamma - 1)(rho e - |rho u|^2 / 2 rho), |u|^2; computed
-    // with the operations of euler.jl:163-175, so staging them per node gives the
-    // values a per-pair evaluation would
-    struct Prim {
-        R u[DIM], b, uu;
+    // EC: rho, b = rho / p (twice Raven's b) and half the velocity; central
+    // Euler: rho, p, the velocity and (v) E + p; advection: q in rho
+    struct Node {
+        R rho, b, u[DIM], v;
     };
-    __device__ static inline Prim prim(const Law<DIM, LAW, R> &law, const R *q)
-    {
-        Prim P;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            P.u[d] = q[1 + d] / q[0];
-        R dot = q[1] * q[1];
-#pragma unroll
-        for (int d = 1; d < DIM; ++d)
-            dot = dot + q[1 + d] * q[1 + d];
-        const R p = law.gm1 * (q[DIM + 1] - dot / (R(2) * q[0]));
-        P.b = q[0] / (R(2) * p);
-        P.uu = P.u[0] * P.u[0];
-#pragma unroll
-        for (int d = 1; d < DIM; ++d)
-            P.uu = P.uu + P.u[d] * P.u[d];
-        return P;
-    }
 
-    // EntropyConservativeFlux (euler.jl:150-184), rows row0 .. row0 + nrows - 1
-    __device__ static inline void ec_rows(const Law<DIM, LAW, R> &law, const R *q1,
-                                          const Prim &P1, const R *q2, const Prim &P2, int row0,
-                                          int nrows, R (*F)[NS])
+    // the values of a node: rho, b (EC) or p, u / 2 (EC) or u
+    __device__ static __forceinline__ void values(const Law<DIM, LAW, R> &law, const R *q, R *x)
     {
-        R uavg[DIM], fr[DIM];
-        const R ravg = (q1[0] + q2[0]) / R(2);
+        x[0] = q[0];
+        if constexpr (!ADV) {
+            const R rinv = R(1) / q[0];
+            R dot = q[1] * q[1];
 #pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            uavg[d] = (P1.u[d] + P2.u[d]) / R(2);
-        const R bavg = (P1.b + P2.b) / R(2);
-        const R u2avg = (P1.uu + P2.uu) / R(2);
-        // the logarithmic means as (a + b) / 2F: rho's taken whole, b's only
-        // through 1 / (2 gm1 blog) = F_b / (2 bavg gm1), which shares
-        // 1 / (2 bavg) with the pressure average
-        const R rlog = ravg / logavg_factor(q1[0], q2[0]);
-        const R Fb = logavg_factor(P1.b, P2.b);
-        const R inv2b = R(1) / (R(2) * bavg);
+            for (int d = 1; d < DIM; ++d)
+                dot = dot + q[1 + d] * q[1 + d];
+            const R p = law.gm1 * (q[DIM + 1] - dot * (R(0.5) * rinv));
+            x[1] = EC ? q[0] / p : p;
 #pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            fr[d] = uavg[d] * rlog;
-        const R pav = ravg * inv2b;
-        const R c = Fb * inv2b * (R(1) / law.gm1) - u2avg / R(2);
-        for (int r = 0; r < nrows; ++r) {
-            const int d = row0 + r;
-            F[r][0] = fr[d];
-#pragma unroll
-            for (int b = 0; b < DIM; ++b)
-                F[r][1 + b] = uavg[d] * fr[b] + (d == b ? pav : R(0));
-            R v = F[r][1] * uavg[0];
-#pragma unroll
-            for (int b = 1; b < DIM; ++b)
-                v = v + F[r][1 + b] * uavg[b];
-            F[r][DIM + 1] = c * fr[d] + v;
+            for (int d = 0; d < DIM; ++d)
+                x[2 + d] = EC ? R(0.5) * (q[1 + d] * rinv) : q[1 + d] * rinv;
         }
     }
 
-    // logavg (numericalfluxes.jl:9-22): the logarithmic mean is (a + b) / (2F),
-    // F = log(zeta) / (2f) = atanh(f) / f with zeta = a / b and
-    // f = (zeta - 1) / (zeta + 1) = (a - b) / (a + b).  Raven takes the series
-    // of F in u = f^2 below the type's epsilon and the logarithm above; here
-    // the series runs up to u < 1e-2, to the term that leaves its remainder
-    // below the type's rounding (u^9 / 19 in FP64, u^5 / 11 in FP32), and
-    // f comes from a - b: as accurate as Raven's form (within 2.2 eps of the
-    // exact mean on 20,000 random pairs, against 2.4 eps), and neighbouring
-    // nodes of a resolved state never reach the logarithm, two divisions
-    // and a log fewer per mean; returns F
-    __device__ static inline R logavg_factor(R a, R b)
+    __device__ static __forceinline__ Node node(const Law<DIM, LAW, R> &law, const R *x)
     {
-        const R f = (a - b) / (a + b);
-        const R u = f * f;
-        R F;
-        if (u < R(1e-2)) {
-            if constexpr (sizeof(R) == 8) {
-                F = R(1) / R(17);
+        Node a;
+        a.rho = x[0];
+        a.b = a.v = R(0);
+        if constexpr (!ADV) {
+            a.b = x[1];
+            R uu = R(0);
 #pragma unroll
-                for (int k = 7; k >= 0; --k)
-                    F = F * u + R(1) / R(2 * k + 1);
-            } else {
-                F = R(1) / R(9);
-#pragma unroll
-                for (int k = 3; k >= 0; --k)
-                    F = F * u + R(1) / R(2 * k + 1);
+            for (int d = 0; d < DIM; ++d) {
+                a.u[d] = x[2 + d];
+                uu = d == 0 ? x[2] * x[2] : uu + x[2 + d] * x[2 + d];
             }
-        } else {
-            F = log(a / b) / (R(2) * f);
+            if constexpr (!EC)
+                a.v = a.b * (law.gamma / law.gm1) + R(0.5) * a.rho * uu;
         }
-        return F;
+        return a;
+    }
+
+    // f#(a, b) along m (GEN), else component 0.  SERIES: which of the log
+    // series (the caller has made sure that every u = f^2 is below its limit),
+    // or -1 for any pair of states.
+    template <int SERIES>
+    __device__ static __forceinline__ void flux(const Law<DIM, LAW, R> &law, const Node &a,
+                                                const Node &b, const R *m, R *F)
+    {
+        if constexpr (ADV) {
+            R un = law.u[0];
+            if constexpr (GEN) {
+                un = law.u[0] * m[0];
+#pragma unroll
+                for (int d = 1; d < DIM; ++d)
+                    un = un + law.u[d] * m[d];
+            }
+            F[0] = R(0.5) * un * (a.rho + b.rho);
+        } else if constexpr (!EC) {
+            R una = a.u[0], unb = b.u[0];
+            if constexpr (GEN) {
+                una = a.u[0] * m[0], unb = b.u[0] * m[0];
+#pragma unroll
+                for (int d = 1; d < DIM; ++d) {
+                    una = una + a.u[d] * m[d];
+                    unb = unb + b.u[d] * m[d];
+                }
+            }
+            una = R(0.5) * una, unb = R(0.5) * unb;
+            const R fa = a.rho * una, fb = b.rho * unb;
+            const R p = R(0.5) * (a.b + b.b);
+            F[0] = fa + fb;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                const R v = fa * a.u[d] + fb * b.u[d];
+                F[1 + d] = GEN ? v + p * m[d] : d == 0 ? v + p : v;
+            }
+            F[DIM + 1] = una * a.v + unb * b.v;
+        } else {
+            // EntropyConservativeFlux (euler.jl:150-184).  With s = a + b and
+            // f = (a - b) / (a + b): rho's logarithmic mean is s_rho / 2F, the
+            // pressure average s_rho / s_b, and the energy flux
+            //   f_rho (1 / (2 gm1 blog) - (u2)avg / 2 + |uavg|^2) + p uavg
+            // = f_rho (2 F_b / (gm1 s_b) + u_a . u_b / 2) + p uavg
+            // with s_b of twice Raven's b.  One reciprocal of s_rho s_b serves
+            // both quotients in FP64; FP32 takes one each (its range is too
+            // small for the product).
+            const R sr = a.rho + b.rho, dr = a.rho - b.rho;
+            const R sb = a.b + b.b, db = a.b - b.b;
+            R isr, isb;
+            if constexpr (sizeof(R) == 8) {
+                const R i = recip(sr * sb);
+                isr = i * sb;
+                isb = i * sr;
+            } else {
+                isr = recip(sr);
+                isb = recip(sb);
+            }
+            const R fr = dr * isr, fb = db * isb;
+            const R ur = fr * fr, ub = fb * fb;
+            R G, Fb;  // 1 / 2F of rho, F of b
+            if constexpr (SERIES < 0) {
+                // the logarithm beyond the series
+                if (ur < R(LogSeries<R>::LIMIT[0]))
+                    G = series_g<R, 0>(ur);
+                else
+                    G = fr / log(a.rho / b.rho);
+                if (ub < R(LogSeries<R>::LIMIT[0]))
+                    Fb = series_f<R, 0>(ub);
+                else
+                    Fb = log(a.b / b.b) / (R(2) * fb);
+            } else {
+                G = series_g<R, SERIES>(ur);
+                Fb = series_f<R, SERIES>(ub);
+            }
+            R ua[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d)
+                ua[d] = a.u[d] + b.u[d];
+            R un = ua[0];
+            if constexpr (GEN) {
+                un = ua[0] * m[0];
+#pragma unroll
+                for (int d = 1; d < DIM; ++d)
+                    un = un + ua[d] * m[d];
+            }
+            const R f0 = un * (sr * G);
+            const R p = sr * isb;
+            R e = (R(2) * a.u[0]) * b.u[0];  // (2 a.u is common to a node's pairs)
+#pragma unroll
+            for (int d = 1; d < DIM; ++d)
+                e = e + (R(2) * a.u[d]) * b.u[d];
+            e = (Fb * isb) * (R(2) / law.gm1) + e;
+            F[0] = f0;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d)
+                F[1 + d] = GEN ? f0 * ua[d] + p * m[d] : d == 0 ? f0 * ua[0] + p : f0 * ua[d];
+            e = f0 * e + p * un;
+            F[DIM + 1] = e;
+        }
     }
 };
 
@@ -160,418 +283,777 @@ template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF>
 struct FD {
     static constexpr int NS = LawInfo<DIM, LAW>::NS;
     static constexpr int NP = IPow<NQ, DIM>::v;
-    static constexpr int NFP = IPow<NQ, DIM - 1>::v;
+    static constexpr int NL = NP / NQ;  // lines per direction, face nodes per face
     static constexpr int NF = 2 * DIM;
-    static constexpr int CPB = fd_cells_per_workgroup(NP);
-    // volume pairs: the Nq (Nq - 1) / 2 symmetric pairs of each line, NL lines
-    // per cell and direction; HL lines per pass through the LDS pair buffer of
-    // at most 36 KB (two 512-thread FP64 workgroups per CU, as the register
-    // bound allows; a smaller FP32 buffer for more workgroups per CU measured
-    // slower: 2.03 against 1.80 ms per stage at Nq = 8)
-    static constexpr int NL = NP / NQ;
-    static constexpr int NPAIR = NQ * (NQ - 1) / 2;
-    static constexpr int BL = CPB * NL;
-    static constexpr int HL_FIT = 36864 / (NPAIR * NS * (int)sizeof(R));
-    static constexpr int HL = HL_FIT < 1 ? 1 : (HL_FIT < BL ? HL_FIT : BL);
-    // the pair buffer is stored line-fastest in rows of HLP values, HLP odd, so
-    // that lanes reading one pair of consecutive lines, or different pairs of
-    // one line, fall in different LDS banks
-    static constexpr int HLP = HL % 2 == 0 ? HL + 1 : HL;
-    static constexpr int THREADS = CPB * NP;
+    static constexpr bool GEN = GEO == GEO_GENERAL;
+    using TP = TwoPoint<DIM, LAW, VF, R, GEN>;
+    static constexpr int C = fd_cells_per_workgroup(DIM, NQ);
+    static constexpr int TASKS = C * DIM * NL;
+    static constexpr int THREADS = (TASKS + 63) / 64 * 64;
+    static constexpr int ITER = (C * NP + THREADS - 1) / THREADS;  // nodes per thread
+    // rows of Nq nodes are padded to an odd length in LDS, so that the lanes
+    // walking x-lines fall in different banks
+    static constexpr int PR = NQ | 1;
+    static constexpr int CS = NL * PR;
+    static constexpr int CMP = C * CS;  // one component of the workgroup's cells
+    // components: rho, b, then u, v, w and (affine) u, v again
+    static constexpr int NC = TP::NV + (GEN || TP::ADV ? 0 : DIM - 1);
+    static constexpr int POOL = CMP * (NC > NS ? NC : NS);
+    // FP64: the line's sums take 2 Nq Ns registers; partners are read from LDS
+    // at every pair instead of being held, so that three waves share a SIMD
+    static constexpr bool REREAD = sizeof(R) == 8 && NQ >= 5;
+    // the faces' states are requested before the pairs where they fit the
+    // registers next to the line's sums (32-bit words)
+    static constexpr bool EARLY = NS * (NQ + 4) * (int)(sizeof(R) / 4) <= 80;
+    // the node kernel's workgroup
+    static constexpr int NODE_C = fd_node_cells(DIM, NQ);
+    static constexpr int NODE_THREADS = (NODE_C * NP + 63) / 64 * 64;
     using S = Stage<DIM, NQ, LAW, R, GEO, FLUX_RUSANOV>;
 };
 
-template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX>
+// P.eprod[workgroup] = the sum of its threads' products (a relaxation stage),
+// compensated, in a fixed order: a butterfly of (sum, compensation) pairs
+// inside each wave (both lanes of a pair form the same sum), then the wave
+// sums in wave order
+template <int THREADS>
+__device__ __forceinline__ void store_product(const StageParams &P, double prod, double pc)
+{
+    __shared__ double red[2 * (THREADS / 64)];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double os = __shfl_xor(prod, off), oc = __shfl_xor(pc, off);
+        comp_add(prod, pc, os, oc);
+    }
+    if ((t & 63) == 0) {
+        red[2 * (t >> 6)] = prod;
+        red[2 * (t >> 6) + 1] = pc;
+    }
+    __syncthreads();
+    if (t == 0) {
+        double sum = red[0], comp = red[1];
+        for (int w = 1; w < THREADS / 64; ++w)
+            comp_add(sum, comp, red[2 * w], red[2 * w + 1]);
+        P.eprod[blockIdx.x] = sum + comp;
+    }
+}
+
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
 __device__ __forceinline__ void fd_stage(const StageParams &P)
 {
     using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
     using S = typename T::S;
-    constexpr int NS = T::NS, NP = T::NP, NFP = T::NFP, NF = T::NF;
-    __shared__ R qs[T::CPB][NS][NP];
-    // entropy-conservative flux: per-node primitives of the line partners
-    constexpr bool EC = VF == FLUX_EC && LAW == LAW_EULER;
-    using TP = TwoPoint<DIM, NS, LAW, VF, R>;
-    using PrimT = typename TP::Prim;
-    __shared__ PrimT ps[EC ? T::CPB : 1][EC ? NP : 1];
+    using TP = typename T::TP;
+    using Node = typename TP::Node;
+    constexpr int NS = T::NS, NP = T::NP, NL = T::NL, NF = T::NF, PR = T::PR, CMP = T::CMP;
+    constexpr bool GEN = T::GEN, ADV = TP::ADV;
+    __shared__ __align__(16) R lds[T::POOL];
     const int t = threadIdx.x;
-    const int c = t / NP, node = t - c * NP;
-    const int64_t e0 = (int64_t)blockIdx.x * T::CPB + c;
-    const bool active = e0 < P.K;
-    // every thread takes part in the pair passes (and a relaxation stage's
-    // workgroup sum): a thread past the last cell repeats the last cell's work
-    // and stores nothing
-    const int64_t e = active ? e0 : P.K - 1;
+    const int64_t cell0 = xcd_remap(blockIdx.x, gridDim.x) * T::C;
     const Law<DIM, LAW, R> law(P);
     const R *qin = static_cast<const R *>(P.q_in);
-    R acc[NS];
+    // cells past the last one repeat its work and store nothing
+    auto cell = [&](int c) {
+        const int64_t e = cell0 + c;
+        return e < P.K ? e : P.K - 1;
+    };
+
+    // ---- phase 0: primitives
     {
-        R q[NS];
+        R q[T::ITER][NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            q[s] = qin[(e * NS + s) * NP + node];
-            qs[c][s][node] = q[s];
+        for (int it = 0; it < T::ITER; ++it) {
+            const int v = t + it * T::THREADS;
+            if (v < T::C * NP) {
+                const int c = v / NP, node = v - c * NP;
+                const R *qe = qin + cell(c) * (NS * NP) + node;
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    q[it][s] = qe[s * NP];
+            }
         }
-        if constexpr (EC)
-            ps[c][node] = TP::prim(law, q);
+#pragma unroll
+        for (int it = 0; it < T::ITER; ++it) {
+            const int v = t + it * T::THREADS;
+            if (v < T::C * NP) {
+                const int c = v / NP, node = v - c * NP;
+                R *x = lds + c * T::CS + node + (PR - NQ) * (node / NQ);
+                R val[TP::NV];
+                TP::values(law, q[it], val);
+#pragma unroll
+                for (int k = 0; k < TP::NV; ++k)
+                    x[k * CMP] = val[k];
+                if constexpr (!GEN && !ADV) {
+#pragma unroll
+                    for (int d = 0; d + 1 < DIM; ++d)
+                        x[(TP::NV + d) * CMP] = val[2 + d];
+                }
+            }
+        }
     }
     __syncthreads();
-    const int ijk[3] = {node % NQ, DIM > 1 ? (node / NQ) % NQ : 0,
-                        DIM > 2 ? node / (NQ * NQ) : 0};
-    const double MJ1 = P.mj[e * NP + node];
-    const double MJI = GEO == GEO_GENERAL ? P.mji[e * NP + node] : 1.0 / MJ1;
-    const R a = R(P.a);
-    R *dq = static_cast<R *>(P.dq);
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-        acc[s] = P.read_dq && !RX ? a * dq[(e * NS + s) * NP + node] : R(0);
 
-    // ---- volume: one direction after another (esvolumeterm_dir!).  Node i's
-    // term from line partner n is MJI_i (D[n,i] G_n - D[i,n] G_i) with
-    // G_x = l_g(x) . f#(q_i, q_n): with f# symmetric, the pair's
-    // H = D[n,i] G_n - D[i,n] G_i serves both ends (+H at i, -H at n), so each
-    // pair is evaluated once (as the reference's :per_dir_symmetric kernel),
-    // by threads packed densely over the workgroup's pairs, and every node
-    // then adds its partners' +-MJI H in partner order from LDS.  The
-    // diagonal term is zero.
-    // the pair buffer; a relaxation stage's workgroup sum reuses it at the end
-    // (and the surface pass's face terms after it)
-    constexpr int HS_BYTES = T::NPAIR * NS * T::HLP * (int)sizeof(R);
-    constexpr int FS_BYTES = T::CPB * NF * NFP * NS * (int)sizeof(R);
-    constexpr int RED_BYTES = RX ? 2 * T::THREADS * (int)sizeof(double) : 0;
-    constexpr int POOL0 = HS_BYTES > FS_BYTES ? HS_BYTES : FS_BYTES;
-    __shared__ __align__(16) char pool[POOL0 > RED_BYTES ? POOL0 : RED_BYTES];
-    R *hs = reinterpret_cast<R *>(pool);
+    // ---- phase 1: a line per lane
+    int dir = t / (T::C * NL);
+    if constexpr (T::C * NL % 64 == 0)
+        dir = __builtin_amdgcn_readfirstlane(dir);  // a wave has one direction
+    const bool line_on = t < T::TASKS && ((P.dir_mask >> dir) & 1);
+    // the line's cell and index, its first node and stride: unpadded, and in
+    // the LDS layout
+    const int nstr = dir == 0 ? 1 : dir == 1 ? NQ : NQ * NQ;
+    const int lstr = dir == 0 ? 1 : dir == 1 ? PR : PR * NQ;
+    struct Line {
+        int c, l, nbase, lbase;
+    };
+    auto line_of = [&](int tt) {
+        Line r;
+        r.c = T::C == 1 ? 0 : (tt - dir * (T::C * NL)) / NL;
+        r.l = tt - dir * (T::C * NL) - r.c * NL;
+        r.nbase = dir == 0 ? r.l * NQ : dir == 1 ? r.l % NQ + (r.l / NQ) * (NQ * NQ) : r.l;
+        r.lbase = r.c * T::CS + (dir == 0   ? r.l * PR
+                                 : dir == 1 ? r.l % NQ + (r.l / NQ) * (PR * NQ)
+                                            : r.l % NQ + (r.l / NQ) * PR);
+        return r;
+    };
+    // (an opaque copy of the thread's index: what is derived from it again
+    // after the pairs need not be held in registers through them)
+    auto fresh = [](int tt) {
+        asm volatile("" : "+v"(tt));
+        return tt;
+    };
+    const int uoff = GEN ? 0 : dir * CMP;
+    R acc[NQ][NS];
+    R scale = R(0);  // dRdX of the line's cell and direction (curved cells: 1)
+    if (line_on) {
+        const Line line = line_of(t);
+        int lbase = line.lbase;
+        const int64_t e = cell(line.c);
+        // the law as the line sees it: its direction first (affine cells)
+        Law<DIM, LAW, R> lawp = law;
+        if constexpr (ADV && !GEN && DIM > 1) {
 #pragma unroll
-    for (int dir = 0; dir < DIM; ++dir) {
-        if (!((P.dir_mask >> dir) & 1))
-            continue;
-        const int id = ijk[dir];
-        int stride = 1;
+            for (int d = 0; d < DIM; ++d)
+                lawp.u[d] = dir == 0   ? law.u[d]
+                            : dir == 1 ? law.u[(d + 1) % DIM]
+                                       : law.u[(d + 2) % DIM];
+        }
+        auto load = [&](int n) {
+            const R *x = lds + lbase + n * lstr;
+            R val[TP::NV];
+            val[0] = x[0];
+            if constexpr (!ADV) {
+                val[1] = x[CMP];
 #pragma unroll
-        for (int d = 0; d < dir; ++d)
-            stride *= NQ;
-        const int myline = c * T::NL + node % stride + (node / (stride * NQ)) * stride;
-        const R mji = R(MJI);
-        // pair order over the lanes: along x, the pairs of one line side by
-        // side (a line's nodes are contiguous); along y and z, one pair of
-        // consecutive lines side by side (lines are contiguous there), so
-        // that lanes read different LDS banks
-        const bool line_major = dir == 0;
-        for (int l0 = 0; l0 < T::BL; l0 += T::HL) {
-            const int nl = T::BL - l0 < T::HL ? T::BL - l0 : T::HL;
-            for (int item = t; item < T::HL * T::NPAIR; item += T::THREADS) {
-                int cl, pr;
-                if (line_major) {
-                    cl = item / T::NPAIR;
-                    pr = item - cl * T::NPAIR;
+                for (int d = 0; d < DIM; ++d)
+                    val[2 + d] = x[uoff + (2 + d) * CMP];
+            }
+            return TP::node(law, val);
+        };
+        // FP32 state reads the FP32 copies of the 3-D geometry (every use
+        // rounds to the state's type)
+        constexpr bool G32 = GEN && DIM == 3 && sizeof(R) == 4;
+        using GT = typename std::conditional<G32, float, double>::type;
+        const GT RV_GLOBAL *vgeo, *sgeo;
+        if constexpr (G32)
+            vgeo = P.vgeo32, sgeo = P.sgeo32;
+        else
+            vgeo = P.vgeo, sgeo = P.sgeo;
+        const int64_t gbase = (e * DIM + dir) * DIM * NP + line.nbase;
+        auto metric = [&](int n, R *lg) {
+#pragma unroll
+            for (int d = 0; d < DIM; ++d)
+                lg[d] = R(vgeo[gbase + n * nstr + d * NP]);
+        };
+        FaceRec rec[2];
+#pragma unroll
+        for (int side = 0; side < 2; ++side)
+            rec[side] = P.faces[e * NF + 2 * dir + side];
+        // uniform tables through the scalar cache: S[i][n] = D[n,i] w_n / w_i -
+        // D[i,n] (affine) and D[i,n] (curved)
+        using Tab = const R __attribute__((address_space(4)));
+        Tab *S_in = (Tab *)(static_cast<const R RV_GLOBAL *>(P.fdtab));
+        Tab *Dtab = S_in + NQ * NQ;
+
+        // the faces the line ends on (surfaceterm!): both ends' states from
+        // memory (the caches hold the cell's own), momentum with the line's
+        // direction first on affine cells
+        R qm[2][NS], qp[2][NS];
+        int l;
+        auto face_states = [&](int tt) {
+            const Line ln = line_of(tt);
+            l = ln.l;
+            lbase = ln.lbase;
+            int comp[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                comp[s] = s;
+            if constexpr (!GEN && !ADV && DIM > 1) {
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    const int k = dir + d;
+                    comp[1 + d] = 1 + (k >= DIM ? k - DIM : k);
+                }
+            }
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                const R *qe = qin + e * (NS * NP) + ln.nbase + (side ? (NQ - 1) * nstr : 0);
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    qm[side][s] = qe[comp[s] * NP];
+                const FaceRec rc = rec[side];
+                if (rc.x != FACE_SELF) {
+                    int64_t off;
+                    if (rc.x >= 0) {
+                        const int fn = rc.y & 7, o = (rc.y >> 3) & 7;
+                        off = (int64_t)rc.x * (NS * NP) +
+                              face_node<DIM, NQ>(fn, orient_node<DIM, NQ>(o, l));
+                    } else {
+                        off = P.explicit_idx[(int64_t)rc.y + l];
+                    }
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+                        qp[side][s] = qin[off + comp[s] * NP];
                 } else {
-                    pr = item / T::HL;
-                    cl = item - pr * T::HL;
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+                        qp[side][s] = qm[side][s];
                 }
-                if (cl >= nl)
+            }
+        };
+        if constexpr (T::EARLY)
+            face_states(t);
+
+        // Which log series serves every pair of the wave's lines: a pair's f is
+        // at most that of the line's extremes.  The extremes are taken on the
+        // leading 32 bits (positive values order as their bits do; a negative
+        // or NaN value fails the test), the largest rounded up.
+        int rough = 0;  // 0: short series, 1: long series, 2: logarithms
+        if constexpr (TP::EC) {
+            constexpr int W = sizeof(R) / 4;  // 32-bit words per value
+            const uint32_t *w = reinterpret_cast<const uint32_t *>(lds) + W * lbase + (W - 1);
+            bool ok[2] = {true, true};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                uint32_t lo = w[W * k * CMP], hi = lo;
+#pragma unroll
+                for (int n = 1; n < NQ; ++n) {
+                    const uint32_t v = w[W * (n * lstr + k * CMP)];
+                    lo = v < lo ? v : lo;
+                    hi = v > hi ? v : hi;
+                }
+                R x0, x1;
+                if constexpr (W == 2) {
+                    x0 = __longlong_as_double((long long)((uint64_t)lo << 32));
+                    x1 = __longlong_as_double((long long)((uint64_t)hi << 32 | 0xffffffffu));
+                } else {
+                    x0 = __uint_as_float(lo);
+                    x1 = __uint_as_float(hi);
+                }
+                const R d = (x1 - x0) * (x1 - x0), s = (x1 + x0) * (x1 + x0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    ok[j] = ok[j] && d < R(LogSeries<R>::LIMIT[j]) * s;
+            }
+            rough = __all(ok[1]) ? 0 : __all(ok[0]) ? 1 : 2;
+        }
+        auto pairs = [&](auto series) {
+            constexpr int SERIES = decltype(series)::value;
+#pragma unroll
+            for (int i = 0; i + 1 < NQ; ++i) {
+                if constexpr (T::REREAD) {
+                    // (an opaque copy of the addresses: partners are read
+                    // again for each i and not kept)
+                    asm volatile("" : "+v"(lbase));
+                }
+                // (an opaque condition ends the basic block: the scheduler
+                // would otherwise hoist later nodes' reads and spill)
+                int go = 1;
+                asm volatile("" : "+s"(go));
+                if (go == 0)
                     continue;
-                int rem = pr, i = 0;
-                while (rem >= NQ - 1 - i) {
-                    rem -= NQ - 1 - i;
-                    ++i;
-                }
-                const int n = i + 1 + rem;
-                const int gl = l0 + cl, pc = gl / T::NL, l = gl - pc * T::NL;
-                const int base = l % stride + (l / stride) * stride * NQ;
-                const int na = base + i * stride, nb = base + n * stride;
-                int64_t pe = (int64_t)blockIdx.x * T::CPB + pc;
-                pe = pe < P.K ? pe : P.K - 1;
-                R qa[NS], qb[NS];
+                const Node a = load(i);
+                R la[DIM];
+                if constexpr (GEN)
+                    metric(i, la);
 #pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    qa[s] = qs[pc][s][na];
-                    qb[s] = qs[pc][s][nb];
-                }
-                const R Din = R(P.Dt[n * NQ + i]);  // D[i, n]
-                const R Dni = R(P.Dt[i * NQ + n]);  // D[n, i]
-                R h[NS];
-                if constexpr (GEO == GEO_GENERAL) {
-                    R F[DIM][NS], la[DIM], lb[DIM];
-                    if constexpr (EC)
-                        TP::ec_rows(law, qa, ps[pc][na], qb, ps[pc][nb], 0, DIM, F);
-                    else
-                        TP::rows(law, qa, qb, 0, DIM, F);
+                for (int n = i + 1; n < NQ; ++n) {
+                    const Node b = load(n);
+                    R F[NS], wi = R(1), wn = R(-1);
+                    if constexpr (GEN) {
+                        R lb[DIM], m[DIM];
+                        metric(n, lb);
+                        const R Dni = Dtab[n * NQ + i], Din = Dtab[i * NQ + n];
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) {
-                        la[d] = R(P.vgeo[((pe * DIM + dir) * DIM + d) * NP + na]);
-                        lb[d] = R(P.vgeo[((pe * DIM + dir) * DIM + d) * NP + nb]);
+                        for (int d = 0; d < DIM; ++d)
+                            m[d] = Dni * lb[d] - Din * la[d];
+                        TP::template flux<SERIES>(lawp, a, b, m, F);
+                    } else {
+                        TP::template flux<SERIES>(lawp, a, b, nullptr, F);
+                        wi = S_in[i * NQ + n], wn = S_in[n * NQ + i];
                     }
 #pragma unroll
                     for (int s = 0; s < NS; ++s) {
-                        R ga = la[0] * F[0][s], gb = F[0][s] * lb[0];
-#pragma unroll
-                        for (int d = 1; d < DIM; ++d) {
-                            ga = ga + la[d] * F[d][s];
-                            gb = gb + F[d][s] * lb[d];
-                        }
-                        h[s] = Dni * gb - Din * ga;
+                        acc[i][s] = i == 0 && n == 1 ? wi * F[s] : acc[i][s] + wi * F[s];
+                        acc[n][s] = i == 0 ? wn * F[s] : acc[n][s] + wn * F[s];
                     }
-                } else {
-                    R F[1][NS];
-                    if constexpr (EC)
-                        TP::ec_rows(law, qa, ps[pc][na], qb, ps[pc][nb], dir, 1, F);
-                    else
-                        TP::rows(law, qa, qb, dir, 1, F);
-                    const double aff = P.affine[pe * DIM + dir];
-                    const R la = R(P.mj[pe * NP + na] * aff), lb = R(P.mj[pe * NP + nb] * aff);
-#pragma unroll
-                    for (int s = 0; s < NS; ++s)
-                        h[s] = Dni * (F[0][s] * lb) - Din * (la * F[0][s]);
                 }
+            }
+        };
+        if (rough == 0) {
+            pairs(std::integral_constant<int, 1>{});
+        } else if (TP::EC && rough == 1) {
+            pairs(std::integral_constant<int, 0>{});
+        } else if constexpr (TP::EC) {
+            // a rolled loop (its indexes are the same on every lane): the
+            // accumulators are addressed by weights that are zero elsewhere
+#pragma unroll
+            for (int n = 0; n < NQ; ++n)
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
-                    hs[(pr * NS + s) * T::HLP + cl] = h[s];
-            }
-            __syncthreads();
-            const int ml = myline - l0;
-            if (ml >= 0 && ml < nl) {
-                for (int n = 0; n < NQ; ++n) {
-                    if (n == id)
-                        continue;
-                    const int lo = id < n ? id : n, hi = id < n ? n : id;
-                    const int pr = lo * (2 * NQ - lo - 1) / 2 + (hi - lo - 1);
-                    const R w = id < n ? mji : -mji;
+                    acc[n][s] = R(0);
+#pragma unroll 1
+            for (int i = 0; i + 1 < NQ; ++i) {
+                const Node a = load(i);
+                R la[DIM];
+                if constexpr (GEN)
+                    metric(i, la);
+#pragma unroll 1
+                for (int n = i + 1; n < NQ; ++n) {
+                    const Node b = load(n);
+                    R F[NS], wi, wn;
+                    if constexpr (GEN) {
+                        R lb[DIM], m[DIM];
+                        metric(n, lb);
+                        const R Dni = Dtab[n * NQ + i], Din = Dtab[i * NQ + n];
 #pragma unroll
-                    for (int s = 0; s < NS; ++s)
-                        acc[s] = acc[s] + w * hs[(pr * NS + s) * T::HLP + ml];
+                        for (int d = 0; d < DIM; ++d)
+                            m[d] = Dni * lb[d] - Din * la[d];
+                        TP::template flux<-1>(lawp, a, b, m, F);
+                        wi = R(1), wn = R(-1);
+                    } else {
+                        TP::template flux<-1>(lawp, a, b, nullptr, F);
+                        wi = S_in[i * NQ + n], wn = S_in[n * NQ + i];
+                    }
+#pragma unroll
+                    for (int k = 0; k < NQ; ++k) {
+                        const R w = k == i ? wi : k == n ? wn : R(0);
+#pragma unroll
+                        for (int s = 0; s < NS; ++s)
+                            acc[k][s] = acc[k][s] + w * F[s];
+                    }
                 }
             }
-            __syncthreads();
+        }
+
+        if constexpr (!T::EARLY)
+            face_states(fresh(t));
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            constexpr int LAST = NQ - 1;
+            const int end = side ? LAST : 0;
+            R nf[NS], lift;
+            R nv[DIM];
+            if constexpr (GEN) {
+                const GT RV_GLOBAL *sg = sgeo + ((e * NF + 2 * dir + side) * (DIM + 1)) * NL + l;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d)
+                    nv[d] = R(sg[d * NL]);
+                lift = R(sg[DIM * NL]);
+            } else {
+                lift = R(P.winv[end]);
+            }
+            if constexpr (SF != FLUX_RUSANOV) {
+                // twopointflux(q-, q+)' n; on an affine face n = +-e_dir
+                static_assert(SF == VF, "the surface flux is Rusanov or the volume form's own");
+                R val[TP::NV], F[NS];
+                TP::values(lawp, qp[side], val);
+                TP::template flux<-1>(lawp, load(end), TP::node(lawp, val), nv, F);
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    nf[s] = GEN || side ? F[s] : -F[s];
+            } else if constexpr (GEN) {
+                S::nflux_general(lawp, nv, qm[side], qp[side], nf);
+            } else {
+                R fm[NS];
+                lawp.flux_row(0, qm[side], fm);
+                S::nflux_axis(lawp, 0, side ? R(1) : R(-1), fm, qm[side], qp[side], nf);
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                acc[end][s] = acc[end][s] - lift * nf[s];
+        }
+        scale = GEN ? R(1) : R(P.affine[e * DIM + dir]);
+    } else {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                acc[n][s] = R(0);
+    }
+
+    // ---- the update's loads, in flight through phase 2
+    const R a = R(P.a), bdt = R(P.b_dt);
+    R *dq = static_cast<R *>(P.dq);
+    R *qo = static_cast<R *>(P.q_out);
+    double prod = 0.0, pc = 0.0;
+    R q[T::ITER][NS], dqo[T::ITER][NS], mji[T::ITER];
+    double mj[T::ITER];
+#pragma unroll
+    for (int it = 0; it < T::ITER; ++it) {
+        const int v = t + it * T::THREADS;
+        const int cc = v / NP, node = v - cc * NP;
+        const int64_t e = cell0 + cc;
+        if (v < T::C * NP && e < P.K) {
+            const int64_t off = e * (NS * NP) + node;
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                q[it][s] = qin[off + s * NP];
+            if (P.read_dq) {
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    dqo[it][s] = load_dq<ST>(dq + off + s * NP);
+            }
+            mji[it] = GEN ? R(P.mji[e * NP + node]) : R(1);
+            mj[it] = RX ? P.mj[e * NP + node] : 0.0;
         }
     }
 
-    // ---- surface (surfaceterm!): each face node's flux is evaluated once, by
-    // threads packed densely over the workgroup's 2 dim Nq^(dim-1) face nodes
-    // per cell (a thread per volume node would run the flux at the width of
-    // the wave for the eight nodes of a cell edge); lift * nf goes to LDS,
-    // m fastest, and every node subtracts its faces' terms in face order
-    // d = 1..dim, f = 1, 2
-    R *fs = reinterpret_cast<R *>(pool);
-    for (int item = t; item < T::CPB * NF * NFP; item += T::THREADS) {
-        const int fc = item / (NF * NFP), r = item - fc * (NF * NFP);
-        const int f = r / NFP, m = r - f * NFP;
-        const int d = f >> 1;
-        if (!((P.dir_mask >> d) & 1))
-            continue;
-        int64_t fe = (int64_t)blockIdx.x * T::CPB + fc;
-        fe = fe < P.K ? fe : P.K - 1;
-        const int side = (f & 1) ? NQ - 1 : 0;
-        int nm;  // the face node's volume node
-        if constexpr (DIM == 1)
-            nm = side;
-        else if constexpr (DIM == 2)
-            nm = d == 0 ? side + NQ * m : m + NQ * side;
-        else
-            nm = d == 0   ? side + NQ * m
-                 : d == 1 ? m % NQ + NQ * side + NQ * NQ * (m / NQ)
-                          : m + NQ * NQ * side;
-        R qm[NS];
+    // ---- phase 2: x, then y, then z
+    const int lbase = line_of(fresh(t)).lbase;
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-            qm[s] = qs[fc][s][nm];
-        const FaceRec rec = P.faces[fe * NF + f];
-        R qp[NS], nf[NS];
-        if (rec.x >= 0) {
-            const int fn = rec.y & 7, o = (rec.y >> 3) & 7;
-            const int nn = face_node<DIM, NQ>(fn, orient_node<DIM, NQ>(o, m));
+    for (int d = 0; d < DIM; ++d) {
+        __syncthreads();
+        if (t < T::TASKS && dir == d) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s)
-                qp[s] = qin[((int64_t)rec.x * NS + s) * NP + nn];
-        } else if (rec.x == FACE_EXPLICIT) {
-            const int64_t off = P.explicit_idx[(int64_t)rec.y + m];
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-                qp[s] = qin[off + s * NP];
-        } else {
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-                qp[s] = qm[s];
-        }
-        R lift;
-        if constexpr (SF != FLUX_RUSANOV) {
-            // twopointflux(q-, q+)' n: on an affine face n = +-e_d, so the
-            // product is row d of the flux with the face's sign
-            using TS = TwoPoint<DIM, NS, LAW, SF, R>;
-            if constexpr (GEO == GEO_AFFINE) {
-                R F[1][NS];
-                if constexpr (SF == FLUX_EC && LAW == LAW_EULER)
-                    TS::ec_rows(law, qm, ps[fc][nm], qp, TS::prim(law, qp), d, 1, F);
-                else
-                    TS::rows(law, qm, qp, d, 1, F);
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    nf[s] = (f & 1) ? F[0][s] : -F[0][s];
-                lift = R(P.affine[fe * DIM + d] * P.winv[side]);
-            } else {
-                const double *sg = P.sgeo + ((fe * NF + f) * (DIM + 1)) * NFP + m;
-                R F[DIM][NS];
-                if constexpr (SF == FLUX_EC && LAW == LAW_EULER)
-                    TS::ec_rows(law, qm, ps[fc][nm], qp, TS::prim(law, qp), 0, DIM, F);
-                else
-                    TS::rows(law, qm, qp, 0, DIM, F);
-#pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    R v = F[0][s] * R(sg[0]);
-#pragma unroll
-                    for (int cc = 1; cc < DIM; ++cc)
-                        v = v + F[cc][s] * R(sg[cc * NFP]);
-                    nf[s] = v;
+            for (int s = 0; s < NS; ++s) {
+                int k = s;
+                if constexpr (!GEN && !ADV && DIM > 1) {
+                    if (s > 0 && s <= DIM)
+                        k = 1 + (s - 1 + d) % DIM;
                 }
-                lift = R(sg[DIM * NFP] * P.mji[fe * NP + nm]);
+                R *x = lds + k * CMP + lbase;
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) {
+                    const R v = GEN ? acc[n][s] : scale * acc[n][s];
+                    x[n * lstr] = d == 0 ? v : x[n * lstr] + v;
+                }
             }
-        } else if constexpr (GEO == GEO_AFFINE) {
-            R fm[NS];
-            law.flux_row(d, qm, fm);
-            S::nflux_axis(law, d, (f & 1) ? R(1) : R(-1), fm, qm, qp, nf);
-            lift = R(P.affine[fe * DIM + d] * P.winv[side]);
-        } else {
-            const double *sg = P.sgeo + ((fe * NF + f) * (DIM + 1)) * NFP + m;
-            R nv[DIM];
-#pragma unroll
-            for (int cc = 0; cc < DIM; ++cc)
-                nv[cc] = R(sg[cc * NFP]);
-            S::nflux_general(law, nv, qm, qp, nf);
-            lift = R(sg[DIM * NFP] * P.mji[fe * NP + nm]);
         }
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-            fs[((fc * NF + f) * NS + s) * NFP + m] = lift * nf[s];
     }
     __syncthreads();
+
+    // ---- phase 3: update
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const int d = f >> 1;
-        if (!((P.dir_mask >> d) & 1))
-            continue;
-        if (ijk[d] != ((f & 1) ? NQ - 1 : 0))
-            continue;
-        int m = 0;
-        if constexpr (DIM == 2)
-            m = d == 0 ? ijk[1] : ijk[0];
-        if constexpr (DIM == 3)
-            m = d == 0 ? ijk[1] + NQ * ijk[2] : d == 1 ? ijk[0] + NQ * ijk[2] : ijk[0] + NQ * ijk[1];
+    for (int it = 0; it < T::ITER; ++it) {
+        const int v = t + it * T::THREADS;
+        const int cc = v / NP, node = v - cc * NP;
+        const int64_t e = cell0 + cc;
+        if (v < T::C * NP && e < P.K) {
+            const int64_t off = e * (NS * NP) + node;
+            const R *x = lds + cc * T::CS + node + (PR - NQ) * (node / NQ);
+            R k[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                k[s] = GEN ? mji[it] * x[s * CMP] : x[s * CMP];
+            if constexpr (RX) {
+                // the dEta term v(q) . k (odesolvers.jl:130-134)
+                double xd[NS], kd[NS];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    xd[s] = (double)q[it][s];
+                    kd[s] = (double)k[s];
+                }
+                double w;
+                if constexpr (DIM == 3)
+                    w = law_entropy_dot_3d<LAW>(xd, kd, P.gamma);
+                else
+                    w = law_entropy_dot<LAW, DIM>(xd, kd, P.gamma);
+                comp_add(prod, pc, mj[it] * w, 0.0);
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const R val = P.read_dq ? a * dqo[it][s] + k[s] : k[s];
+                store_out<ST>(val, dq + off + s * NP);
+                if (P.write_q)
+                    store_out<ST>(R(q[it][s] + bdt * val), qo + off + s * NP);
+            }
+        }
+    }
+    if constexpr (RX)
+        store_product<T::THREADS>(P, prod, pc);
+}
+
+// A lane per node, which evaluates the fluxes with its dim (Nq - 1) line
+// partners itself: each pair twice, but in short code, with no sums to move
+// between directions and one barrier.
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
+__device__ __forceinline__ void fd_stage_node(const StageParams &P)
+{
+    using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
+    using S = typename T::S;
+    using TP = typename T::TP;
+    constexpr int NS = T::NS, NP = T::NP, NL = T::NL, NF = T::NF, NV = TP::NV;
+    constexpr bool GEN = T::GEN;
+    __shared__ R lds[NV][T::NODE_THREADS];
+    const int t = threadIdx.x;
+    const int c = t / NP, node = t - c * NP;
+    const int64_t e = xcd_remap(blockIdx.x, gridDim.x) * T::NODE_C + c;
+    const bool active = c < T::NODE_C && e < P.K;
+    const Law<DIM, LAW, R> law(P);
+    const R *qin = static_cast<const R *>(P.q_in);
+    R *dq = static_cast<R *>(P.dq);
+    R *qo = static_cast<R *>(P.q_out);
+    const int64_t off = e * (NS * NP) + node;
+    const int ijk[3] = {node % NQ, DIM > 1 ? (node / NQ) % NQ : 0, DIM > 2 ? node / (NQ * NQ) : 0};
+    constexpr bool G32 = GEN && DIM == 3 && sizeof(R) == 4;
+    using GT = typename std::conditional<G32, float, double>::type;
+    const GT RV_GLOBAL *vgeo, *sgeo;
+    if constexpr (G32)
+        vgeo = P.vgeo32, sgeo = P.sgeo32;
+    else
+        vgeo = P.vgeo, sgeo = P.sgeo;
+
+    // the node's own loads, and the neighbour states of the faces it lies on
+    // (one per direction: Nq > 1)
+    R q[NS], x[NV], qp[DIM][NS], dqo[NS], mji = R(1);
+    double mj = 0.0;
+    bool on_face[DIM];
+    int side[DIM], m[DIM];
+    if (active) {
+        FaceRec rec[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            side[d] = ijk[d] == NQ - 1;
+            on_face[d] = ((P.dir_mask >> d) & 1) && (side[d] || ijk[d] == 0);
+            m[d] = DIM == 1   ? 0
+                   : DIM == 2 ? ijk[1 - d]
+                   : d == 0   ? ijk[1] + NQ * ijk[2]
+                   : d == 1   ? ijk[0] + NQ * ijk[2]
+                              : ijk[0] + NQ * ijk[1];
+            if (on_face[d])
+                rec[d] = P.faces[e * NF + 2 * d + side[d]];
+        }
 #pragma unroll
         for (int s = 0; s < NS; ++s)
-            acc[s] = acc[s] - fs[((c * NF + f) * NS + s) * NFP + m];
-    }
-    // the node's own state back from LDS (not held in registers through the
-    // pair and face passes)
-    R q1[NS];
+            q[s] = qin[off + s * NP];
+        if (P.read_dq) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
-        q1[s] = qs[c][s][node];
-
-    // ---- update
-    if constexpr (RX) {
-        // dq .*= rka; dq .+= k; the dEta term v(q) . k (odesolvers.jl:130-134)
-        double x[NS], kk[NS];
+            for (int s = 0; s < NS; ++s)
+                dqo[s] = load_dq<ST>(dq + off + s * NP);
+        }
+        if constexpr (GEN)
+            mji = R(P.mji[e * NP + node]);
+        if constexpr (RX)
+            mj = P.mj[e * NP + node];
+        TP::values(law, q, x);
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+            lds[k][t] = x[k];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+            if (on_face[d]) {
+                int64_t o = off;  // a self-mapped face: q+ = q-
+                if (rec[d].x >= 0)
+                    o = (int64_t)rec[d].x * (NS * NP) +
+                        face_node<DIM, NQ>(rec[d].y & 7,
+                                           orient_node<DIM, NQ>((rec[d].y >> 3) & 7, m[d]));
+                else if (rec[d].x == FACE_EXPLICIT)
+                    o = P.explicit_idx[(int64_t)rec[d].y + m[d]];
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    qp[d][s] = qin[o + s * NP];
+            }
+    }
+    __syncthreads();
+    double prod = 0.0, pc = 0.0;
+    if (active) {
+        const typename TP::Node a = TP::node(law, x);
+        const R *tab = static_cast<const R *>(P.fdtab);
+        R k[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            k[s] = R(0);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            if (!((P.dir_mask >> d) & 1))
+                continue;
+            // the line's direction first (affine cells form component 0)
+            auto turned = [&](const typename TP::Node &b) {
+                typename TP::Node r = b;
+                if constexpr (!GEN) {
+#pragma unroll
+                    for (int j = 0; j < DIM; ++j)
+                        r.u[j] = b.u[(d + j) % DIM];
+                }
+                return r;
+            };
+            Law<DIM, LAW, R> lawd = law;
+            if constexpr (!GEN) {
+#pragma unroll
+                for (int j = 0; j < DIM; ++j)
+                    lawd.u[j] = law.u[(d + j) % DIM];
+            }
+            const typename TP::Node ad = turned(a);
+            const int i = ijk[d];
+            const int stride = d == 0 ? 1 : d == 1 ? NQ : NQ * NQ;
+            const int64_t g = ((e * DIM + d) * DIM) * NP + node;
+            R la[DIM], kd[NS];
+            if constexpr (GEN) {
+#pragma unroll
+                for (int j = 0; j < DIM; ++j)
+                    la[j] = R(vgeo[g + j * NP]);
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                kd[s] = R(0);
+            // (two partners in flight: a wave's chain is what small grids wait for)
+#pragma unroll 2
+            for (int it = 0; it < NQ - 1; ++it) {
+                R y[NV], F[NS], mv[DIM], w = R(1);
+                const int n = it + (it >= i);
+                const int to = (n - i) * stride;
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+                    y[j] = lds[j][t + to];
+                if constexpr (GEN) {
+                    const R *D = tab + NQ * NQ;
+                    const R Dni = D[n * NQ + i], Din = D[i * NQ + n];
+#pragma unroll
+                    for (int j = 0; j < DIM; ++j)
+                        mv[j] = Dni * R(vgeo[g + to + j * NP]) - Din * la[j];
+                } else {
+                    w = tab[i * NQ + n];
+                }
+                TP::template flux<-1>(lawd, ad, turned(TP::node(law, y)), mv, F);
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    kd[s] = kd[s] + w * F[s];
+            }
+            if (on_face[d]) {
+                R nf[NS], nv[DIM], lift;
+                if constexpr (GEN) {
+                    const GT RV_GLOBAL *sg =
+                        sgeo + ((e * NF + 2 * d + side[d]) * (DIM + 1)) * NL + m[d];
+#pragma unroll
+                    for (int j = 0; j < DIM; ++j)
+                        nv[j] = R(sg[j * NL]);
+                    lift = R(sg[DIM * NL]);
+                } else {
+                    lift = R(P.winv[i]);
+                }
+                // the states with the direction's momentum first (affine cells)
+                R qm[NS], qq[NS];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const int o = GEN || TP::ADV || s == 0 || s > DIM ? s : 1 + (d + s - 1) % DIM;
+                    qm[s] = q[o];
+                    qq[s] = qp[d][o];
+                }
+                if constexpr (SF != FLUX_RUSANOV) {
+                    R y[NV], F[NS];
+                    TP::values(lawd, qq, y);
+                    TP::template flux<-1>(lawd, ad, TP::node(lawd, y), nv, F);
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+                        nf[s] = GEN || side[d] ? F[s] : -F[s];
+                } else if constexpr (GEN) {
+                    S::nflux_general(lawd, nv, qm, qq, nf);
+                } else {
+                    R fm[NS];
+                    lawd.flux_row(0, qm, fm);
+                    S::nflux_axis(lawd, 0, side[d] ? R(1) : R(-1), fm, qm, qq, nf);
+                }
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    kd[s] = kd[s] - lift * nf[s];
+            }
+            const R scale = GEN ? R(1) : R(P.affine[e * DIM + d]);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const int o = GEN || TP::ADV || s == 0 || s > DIM ? s : 1 + (d + s - 1) % DIM;
+                k[o] = k[o] + scale * kd[s];
+            }
+        }
+        const R ca = R(P.a), bdt = R(P.b_dt);
+        if constexpr (GEN) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                k[s] = mji * k[s];
+        }
+        if constexpr (RX) {
+            // the dEta term v(q) . k (odesolvers.jl:130-134)
+            double xd[NS], kd[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                xd[s] = (double)q[s];
+                kd[s] = (double)k[s];
+            }
+            if constexpr (DIM == 3)
+                prod = mj * law_entropy_dot_3d<LAW>(xd, kd, P.gamma);
+            else
+                prod = mj * law_entropy_dot<LAW, DIM>(xd, kd, P.gamma);
+        }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            x[s] = (double)q1[s];
-            kk[s] = (double)acc[s];
-            if (P.read_dq)
-                acc[s] = a * dq[(e * NS + s) * NP + node] + acc[s];
-        }
-        double prod = 0.0;
-        if constexpr (DIM == 3)
-            prod = active ? MJ1 * law_entropy_dot_3d<LAW>(x, kk, P.gamma) : 0.0;
-        else
-            prod = active ? MJ1 * law_entropy_dot<LAW, DIM>(x, kk, P.gamma) : 0.0;
-        double pc = 0.0;  // compensation of prod
-        // the workgroup's sum, compensated: a fixed tree over the threads of
-        // (sum, compensation) pairs, each addition's rounding error (TwoSum,
-        // exact and symmetric in its operands) carried in the compensation;
-        // in the pair buffer, once every thread has read its face terms
-        double *red = reinterpret_cast<double *>(pool);
-        __syncthreads();
-        if constexpr (T::THREADS % 64 == 0) {
-            // whole waves: a butterfly inside each wave (both lanes of a pair
-            // form the same sum), then the wave sums in wave order
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const double os = __shfl_xor(prod, off), oc = __shfl_xor(pc, off);
-                comp_add(prod, pc, os, oc);
-            }
-            if ((t & 63) == 0) {
-                red[2 * (t >> 6)] = prod;
-                red[2 * (t >> 6) + 1] = pc;
-            }
-            __syncthreads();
-            if (t == 0) {
-                double sum = red[0], c = red[1];
-                for (int w = 1; w < T::THREADS / 64; ++w)
-                    comp_add(sum, c, red[2 * w], red[2 * w + 1]);
-                P.eprod[blockIdx.x] = sum + c;
-            }
-        } else {
-            red[2 * t] = prod;
-            red[2 * t + 1] = pc;
-            __syncthreads();
-            for (int w = 256; w > 0; w >>= 1) {
-                if (t < w && t + w < T::THREADS) {
-                    double sum = red[2 * t], c = red[2 * t + 1];
-                    comp_add(sum, c, red[2 * (t + w)], red[2 * (t + w) + 1]);
-                    red[2 * t] = sum;
-                    red[2 * t + 1] = c;
-                }
-                __syncthreads();
-            }
-            if (t == 0)
-                P.eprod[blockIdx.x] = red[0] + red[1];
+            const R val = P.read_dq ? ca * dqo[s] + k[s] : k[s];
+            store_out<ST>(val, dq + off + s * NP);
+            if (P.write_q)
+                store_out<ST>(R(q[s] + bdt * val), qo + off + s * NP);
         }
     }
-    if (!active)
-        return;
-    const R bdt = R(P.b_dt);
-    R *qo = static_cast<R *>(P.q_out);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        dq[(e * NS + s) * NP + node] = acc[s];
-        if (P.write_q)
-            qo[(e * NS + s) * NP + node] = q1[s] + bdt * acc[s];
+    if constexpr (RX)
+        store_product<T::NODE_THREADS>(P, prod, pc);
+}
+
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF>
+constexpr int fd_waves_per_simd()
+{
+    return sizeof(R) == 8 ? (GEO == GEO_GENERAL && NQ >= 6 ? 2 : 3) : 4;
+}
+
+// (RX: the relaxation stage)
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
+__global__ void __launch_bounds__((FD<DIM, NQ, LAW, R, GEO, VF, SF>::THREADS))
+    __attribute__((amdgpu_waves_per_eu(fd_waves_per_simd<DIM, NQ, LAW, R, GEO, VF, SF>())))
+        dg_fd_line_kernel(const StageParams P)
+{
+    fd_stage<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>(P);
+}
+
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
+__global__ void __launch_bounds__((FD<DIM, NQ, LAW, R, GEO, VF, SF>::NODE_THREADS))
+    dg_fd_node_kernel(const StageParams P)
+{
+    fd_stage_node<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>(P);
+}
+
+template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
+void launch_fd_st(const StageParams &P, hipStream_t st)
+{
+    using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
+    if constexpr (fd_has_line_kernel(DIM, LAW, VF)) {
+        if (fd_by_line(DIM, NQ, LAW, (int)sizeof(R), VF, P.K)) {
+            hipLaunchKernelGGL((dg_fd_line_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>),
+                               dim3((unsigned)((P.K + T::C - 1) / T::C)), dim3(T::THREADS), 0, st,
+                               P);
+            return;
+        }
     }
-}
-
-// A 512-thread workgroup (two waves per SIMD) is held to 128 VGPRs so that two
-// workgroups share a CU: measured on MI355X at Nq = 8 (3-D Euler, entropy
-// conservative, FP64) 3.6 ms per stage against 5.0 ms at the compiler's own
-// 140 VGPRs (one workgroup per CU), a few spilled registers included
-template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF>
-__global__ void __launch_bounds__(512)
-    __attribute__((amdgpu_waves_per_eu(FD<DIM, NQ, LAW, R, GEO, VF, SF>::THREADS == 512 ? 4 : 1)))
-        dg_fd_kernel(const StageParams P)
-{
-    fd_stage<DIM, NQ, LAW, R, GEO, VF, SF, false>(P);
-}
-
-// the relaxation stage, under the same register bound
-template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF>
-__global__ void __launch_bounds__(512)
-    __attribute__((amdgpu_waves_per_eu(FD<DIM, NQ, LAW, R, GEO, VF, SF>::THREADS == 512 ? 4 : 1)))
-        dg_fd_relax_kernel(const StageParams P)
-{
-    fd_stage<DIM, NQ, LAW, R, GEO, VF, SF, true>(P);
+    hipLaunchKernelGGL((dg_fd_node_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>),
+                       dim3((unsigned)((P.K + T::NODE_C - 1) / T::NODE_C)), dim3(T::NODE_THREADS),
+                       0, st, P);
 }
 
 template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX>
 int launch_fd(const StageParams &P, void *stream, int)
 {
-    using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
     if (P.K <= 0)
         return 0;
-    const int64_t blocks = (P.K + T::CPB - 1) / T::CPB;
-    if constexpr (RX)
-        hipLaunchKernelGGL((dg_fd_relax_kernel<DIM, NQ, LAW, R, GEO, VF, SF>),
-                           dim3((unsigned)blocks), dim3(T::THREADS), 0,
-                           static_cast<hipStream_t>(stream), P);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (P.streaming)
+        launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, st);
     else
-        hipLaunchKernelGGL((dg_fd_kernel<DIM, NQ, LAW, R, GEO, VF, SF>), dim3((unsigned)blocks),
-                           dim3(T::THREADS), 0, static_cast<hipStream_t>(stream), P);
+        launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 0>(P, st);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
