@@ -179,8 +179,9 @@ struct TwoPoint {
     }
 
     // f#(a, b) along m (GEN), else component 0.  SERIES: which of the log
-    // series (the caller has made sure that every u = f^2 is below its limit),
-    // or -1 for any pair of states.
+    // series (the caller has made sure that every u = f^2 is below its limit,
+    // and that rho b is far from the type's range), or -1 for any pair of
+    // states.
     template <int SERIES>
     __device__ static __forceinline__ void flux(const Law<DIM, LAW, R> &law, const Node &a,
                                                 const Node &b, const R *m, R *F)
@@ -220,13 +221,13 @@ struct TwoPoint {
             // pressure average s_rho / s_b, and the energy flux
             //   f_rho (1 / (2 gm1 blog) - (u2)avg / 2 + |uavg|^2) + p uavg
             // = f_rho (2 F_b / (gm1 s_b) + u_a . u_b / 2) + p uavg
-            // with s_b of twice Raven's b.  One reciprocal of s_rho s_b serves
-            // both quotients in FP64; FP32 takes one each (its range is too
-            // small for the product).
+            // with s_b of twice Raven's b.  In FP64 one reciprocal of s_rho s_b
+            // serves both quotients where the caller knows the product's range
+            // (SERIES >= 0); FP32's range is too small for the product.
             const R sr = a.rho + b.rho, dr = a.rho - b.rho;
             const R sb = a.b + b.b, db = a.b - b.b;
             R isr, isb;
-            if constexpr (sizeof(R) == 8) {
+            if constexpr (sizeof(R) == 8 && SERIES >= 0) {
                 const R i = recip(sr * sb);
                 isr = i * sb;
                 isb = i * sr;
@@ -532,6 +533,7 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
             constexpr int W = sizeof(R) / 4;  // 32-bit words per value
             const uint32_t *w = reinterpret_cast<const uint32_t *>(lds) + W * lbase + (W - 1);
             bool ok[2] = {true, true};
+            R least = R(1), most = R(1);  // of rho times b (see TwoPoint::flux)
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 uint32_t lo = w[W * k * CMP], hi = lo;
@@ -549,11 +551,15 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
                     x0 = __uint_as_float(lo);
                     x1 = __uint_as_float(hi);
                 }
+                least = least * x0, most = most * x1;
                 const R d = (x1 - x0) * (x1 - x0), s = (x1 + x0) * (x1 + x0);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     ok[j] = ok[j] && d < R(LogSeries<R>::LIMIT[j]) * s;
             }
+            if constexpr (W == 2)
+                ok[0] = ok[0] && least > R(1e-290) && most < R(1e290);
+            ok[1] = ok[1] && ok[0];
             rough = __all(ok[1]) ? 0 : __all(ok[0]) ? 1 : 2;
         }
         auto pairs = [&](auto series) {
