@@ -551,14 +551,15 @@ __global__ void round_to_f32_kernel(const double *__restrict__ src, float *__res
         dst[i] = (float)src[i];
 }
 
-// The FP32 copies of the general geometry (and MJ) that the 3-D column kernel
-// of an FP32 handle reads (StageParams::vgeo32 ...), made again after every
+// The FP32 copies of the general geometry (and MJ) that the 2-D and 3-D stage
+// kernels of an FP32 handle read (StageParams::vgeo32 ...), made again after every
 // change of the FP64 arrays.
 int refresh_geo32(rv_handle *h)
 {
-    if (!(h->dtype == RV_F32 && h->geo == GEO_GENERAL && h->dim == 3) || h->K <= 0)
+    if (!(h->dtype == RV_F32 && h->geo == GEO_GENERAL && h->dim >= 2) || h->K <= 0)
         return RV_OK;
-    const int64_t nv = h->K * 9 * h->Np, nm = h->K * h->Np, ns = h->K * 6 * 4 * h->nfp;
+    const int64_t nv = h->K * h->dim * h->dim * h->Np, nm = h->K * h->Np,
+                  ns = h->K * 2 * h->dim * (h->dim + 1) * h->nfp;
     int rc;
     if (!h->vgeo32 && ((rc = dalloc(h, &h->vgeo32, nv)) || (rc = dalloc(h, &h->mji32, nm)) ||
                        (rc = dalloc(h, &h->sgeo32, ns)) || (rc = dalloc(h, &h->mj32, nm))))
@@ -1278,12 +1279,12 @@ int rv_get_info(const rv_handle *h, rv_info *info)
     info->device_bytes = h->device_bytes;
     // compulsory traffic per node: read q, [read dq], write dq, write q; plus
     // per-node geometry (wJ*dRdX, 1/wJ) and per face-node (n, wsJ) when the
-    // cells are not affine, FP64 except for the 3-D weak form of FP32
-    // handles, whose stage reads the FP32 copies; affine geometry is per cell
+    // cells are not affine, FP64 except for the 2-D and 3-D stages of FP32
+    // handles, which read the FP32 copies; affine geometry is per cell
     // (~0 per node)
     int64_t geo = 0;
     if (h->geo == GEO_GENERAL) {
-        const int gb = h->dtype == RV_F32 && h->dim == 3 && h->vflux == 0 ? 4 : 8;
+        const int gb = h->dtype == RV_F32 && h->dim >= 2 ? 4 : 8;
         geo = nodes * (h->dim * h->dim + 1) * gb + h->K * 2 * h->dim * h->nfp * (h->dim + 1) * gb;
     }
     info->stage_bytes = 4 * info->state_bytes + geo;

@@ -63,9 +63,9 @@ struct StageParams {
     const double RV_GLOBAL *mji;   // (K, Np)
     const double RV_GLOBAL *mj;    // (K, Np) = wJ
     const double RV_GLOBAL *sgeo;  // (K, 2dim, dim+1, Nfp): n_c ..., wsJ
-    // FP32 handles, 3-D general cells: vgeo, mji and sgeo rounded to FP32 once
-    // (the 3-D column kernel rounds every use of them to the state type, so
-    // reading these gives the same results with half the geometry bytes)
+    // FP32 handles, 2-D and 3-D general cells: vgeo, mji, sgeo and mj rounded to
+    // FP32 once (the stage kernels round every use of them to the state type,
+    // so reading these gives the same results with half the geometry bytes)
     const float RV_GLOBAL *vgeo32;
     const float RV_GLOBAL *mji32;
     const float RV_GLOBAL *sgeo32;

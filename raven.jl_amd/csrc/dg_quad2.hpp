@@ -1,14 +1,10 @@
-// Fused 2-D DGSEM stage kernel on affine cells for gfx950: a lane per node.
-//
-// Same operator and the same arithmetic, operation for operation, as the
-// pencil kernel of dg_kernels.hpp (Raven's weak-form volume term, Rusanov /
-// central surface term, LSRK update: dgsem.jl:257-348, 733-784,
-// odesolvers.jl:55-57), so the two give bit-identical results; what changes
-// is the memory access pattern:
+// Fused 2-D DGSEM stage kernel for gfx950: a lane per node.  Raven's weak-form
+// volume term, Rusanov / central surface term and LSRK update
+// (dgsem.jl:257-348, 733-784, odesolvers.jl:55-57):
 //
 //  * lane (i, j) of a cell owns node i + Nq j: q and dq_old are read, and dq
-//    and q_out written, with lane-contiguous addresses (the pencil kernel's
-//    x-pencils are strided by Nq), and q stays in registers for the update;
+//    and q_out written, with lane-contiguous addresses, and q stays in
+//    registers for the update;
 //  * each lane evaluates both flux rows at its node and publishes them in LDS,
 //    x-fluxes in node order and y-fluxes transposed, so that the two
 //    derivative sums a lane needs each read one contiguous row;
@@ -23,8 +19,15 @@
 //    its own); the batches' work-list kernel uses G = 1;
 //  * light cells (advection, FP32 Euler) give a lane V = 4 or 2 nodes, one in
 //    each of V sets of cells, all requested before the first wait: a wave
-//    then has V times the bytes in flight.
+//    then has V times the bytes in flight;
+//  * curved cells publish contravariant fluxes and lifted numerical fluxes.
+//    Bound by memory: on 200^2 warped cells of Nq = 6 an FP64 Euler stage
+//    takes 41.5 us (6.0 TB/s, out of the Infinity Cache; a lane per pencil,
+//    whose x-pencils are strided, took 83.6 us).
 #pragma once
+
+#include <type_traits>
+
 
 #include "dg_kernels.hpp"
 
@@ -74,13 +77,22 @@ constexpr int quad2_nodes_per_lane()
 // [cell0 + v CPS, cell0 + (v + 1) CPS).  gl is the lane's index in the group
 // (0 .. 64 G - 1) and glds the group's slab, whose spare must hold zeros
 // (quad2_clear_spare) when the group starts.
-template <int NQ, int LAW, typename R, int FLUX, int ST, int G, int V>
+template <int NQ, int LAW, typename R, int FLUX, int ST, int G, int V, int GEO = GEO_AFFINE>
 __device__ __attribute__((always_inline)) inline void quad2_group(const StageParams &P,
                                                                   int64_t cell0, R *glds, int gl)
 {
     using Q = Quad2<NQ, LAW, R, FLUX, G, V>;
-    using S = Stage<2, NQ, LAW, R, GEO_AFFINE, FLUX>;
+    using S = Stage<2, NQ, LAW, R, GEO, FLUX>;
     constexpr int NS = Q::NS, NP = Q::NP;
+    constexpr bool GEN = GEO == GEO_GENERAL;
+    // FP32 state reads the FP32 copies of the geometry
+    constexpr bool G32 = GEN && sizeof(R) == 4;
+    using GT = typename std::conditional<G32, float, double>::type;
+    const GT RV_GLOBAL *vgeo, *sgeo, *mjip;
+    if constexpr (G32)
+        vgeo = P.vgeo32, sgeo = P.sgeo32, mjip = P.mji32;
+    else
+        vgeo = P.vgeo, sgeo = P.sgeo, mjip = P.mji;
     const Law<2, LAW, R> law(P);
     const R *qin = static_cast<const R *>(P.q_in);
     R *dqp = static_cast<R *>(P.dq);
@@ -102,6 +114,7 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
     // the node's state and dq_old, the cell scales, and the operator rows and
     // lift weights of the node (requested before the first wait)
     R q[V][NS], dqo[V][NS], sx[V], sy[V], mx[NQ], my[NQ];
+    R geo[V][4], mji[V];  // curved cells: wJ dRdX and 1 / (wJ) of the node
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         sx[v] = sy[v] = R(0);
@@ -115,13 +128,20 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
                     dqo[v][s] = load_dq<ST>(dqp + off[v] + s * NP);
             }
             const int64_t e = cell0 + v * Q::CPS + c;
-            sx[v] = R(P.affine[e * 2 + 0]);
-            sy[v] = R(P.affine[e * 2 + 1]);
+            if constexpr (GEN) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    geo[v][g] = R(vgeo[(e * 4 + g) * NP + node]);
+                mji[v] = R(mjip[e * NP + node]);
+            } else {
+                sx[v] = R(P.affine[e * 2 + 0]);
+                sy[v] = R(P.affine[e * 2 + 1]);
+            }
         }
     }
     R wx = R(0), wy = R(0);
     if (active[0]) {
-        const double *M = P.Dw;
+        const double *M = GEN ? P.Dt : P.Dw;
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
             mx[n] = R(M[i * NQ + n]);
@@ -132,6 +152,7 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
     }
     // face nodes: own and neighbour state (face record first)
     R qm[V][Q::FPASS][NS], qp[V][Q::FPASS][NS];
+    R sg[V][Q::FPASS][3];  // curved cells: n and wsJ of the face node
 #pragma unroll
     for (int v = 0; v < V; ++v)
 #pragma unroll
@@ -148,6 +169,11 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
                 for (int s = 0; s < NS; ++s)
                     qm[v][ps][s] = qe[s * NP];
                 S::neighbour_state(P, qin, fe, f, p, qm[v][ps], qp[v][ps]);
+                if constexpr (GEN) {
+#pragma unroll
+                    for (int g = 0; g < 3; ++g)
+                        sg[v][ps][g] = R(sgeo[((fe * 4 + f) * 3 + g) * NQ + p]);
+                }
             }
         }
     // flux rows at the node, published for the derivative sums
@@ -155,8 +181,19 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
     for (int v = 0; v < V; ++v)
         if (active[v]) {
             R fx[NS], fy[NS];
-            law.flux_row(0, q[v], fx);
-            law.flux_row(1, q[v], fy);
+            if constexpr (GEN) {
+                // contravariant fluxes
+                R F[2][NS];
+                law.flux_all(q[v], F);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    fx[s] = geo[v][0] * F[0][s] + geo[v][1] * F[1][s];
+                    fy[s] = geo[v][2] * F[0][s] + geo[v][3] * F[1][s];
+                }
+            } else {
+                law.flux_row(0, q[v], fx);
+                law.flux_row(1, q[v], fy);
+            }
             R *cl = glds + Q::SPARE_LEN + v * Q::PART + c * (NS * NP);
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
@@ -181,7 +218,13 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
                 // law's private arrays (scratch memory)
                 R fm[NS], nf[NS];
                 const R sgn = (f & 1) ? R(1) : R(-1);
-                if (d == 0) {
+                if constexpr (GEN) {
+                    // published with its lift weight
+                    S::nflux_general(law, sg[v][ps], qm[v][ps], qp[v][ps], nf);
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+                        nf[s] = sg[v][ps][2] * nf[s];
+                } else if (d == 0) {
                     law.flux_row(0, qm[v][ps], fm);
                     S::nflux_axis(law, 0, sgn, fm, qm[v][ps], qp[v][ps], nf);
                 } else {
@@ -221,8 +264,12 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
 #pragma unroll
                 for (int n = 1; n < NQ; ++n)
                     vx = vx + mx[n] * row[n];
-                vx = vx - wx * glds[bx + s];
-                vx = sx[v] * vx;
+                if constexpr (GEN) {
+                    vx = vx - glds[bx + s];
+                } else {
+                    vx = vx - wx * glds[bx + s];
+                    vx = sx[v] * vx;
+                }
             }
             if (ony) {
                 const R *row = cl + Q::FYO + s * NP + i * NQ;
@@ -230,10 +277,14 @@ __device__ __attribute__((always_inline)) inline void quad2_group(const StagePar
 #pragma unroll
                 for (int n = 1; n < NQ; ++n)
                     vy = vy + my[n] * row[n];
-                vy = vy - wy * glds[by + s];
-                vy = sy[v] * vy;
+                if constexpr (GEN) {
+                    vy = vy - glds[by + s];
+                } else {
+                    vy = vy - wy * glds[by + s];
+                    vy = sy[v] * vy;
+                }
             }
-            const R tot = vx + vy;
+            const R tot = GEN ? mji[v] * (vx + vy) : vx + vy;
             R val = tot;
             if (P.read_dq)
                 val = a * dqo[v][s] + tot;
@@ -255,7 +306,7 @@ __device__ inline void quad2_clear_spare(R *glds, int gl)
 
 // Single operator: a workgroup of wpb waves holds wpb / G groups (G > 1:
 // wpb = G, one group).
-template <int NQ, int LAW, typename R, int FLUX, int ST, int G, int V>
+template <int NQ, int LAW, typename R, int FLUX, int ST, int G, int V, int GEO>
 __global__ void __launch_bounds__(256) dg_quad2_kernel(const StageParams P)
 {
     using Q = Quad2<NQ, LAW, R, FLUX, G, V>;
@@ -266,14 +317,17 @@ __global__ void __launch_bounds__(256) dg_quad2_kernel(const StageParams P)
     const int64_t blk = xcd_remap(blockIdx.x, gridDim.x);
     R *glds = reinterpret_cast<R *>(dg_lds) + grp * Q::SLAB;
     quad2_clear_spare(glds, gl);
-    quad2_group<NQ, LAW, R, FLUX, ST, G, V>(P, (blk * gpb + grp) * Q::CELLS, glds, gl);
+    quad2_group<NQ, LAW, R, FLUX, ST, G, V, GEO>(P, (blk * gpb + grp) * Q::CELLS, glds, gl);
 }
 
-template <int NQ, int LAW, typename R, int FLUX>
+template <int NQ, int LAW, typename R, int FLUX, int GEO>
 int launch_quad2(const StageParams &P, void *stream, int wpb)
 {
     constexpr int G = quad2_group_waves<NQ>();
-    constexpr int V = quad2_nodes_per_lane<LAW, R>();
+    // (curved cells: one node per lane, whose metric terms are bytes enough in
+    // flight: 2 took 44 to 51 us against 41 to 46 us per FP64 Euler stage of
+    // 1.4 to 1.6 M nodes, advection likewise)
+    constexpr int V = GEO == GEO_GENERAL ? 1 : quad2_nodes_per_lane<LAW, R>();
     using Q = Quad2<NQ, LAW, R, FLUX, G, V>;
     if (P.K <= 0)
         return 0;
@@ -287,10 +341,10 @@ int launch_quad2(const StageParams &P, void *stream, int wpb)
     const size_t lds = (size_t)gpb * Q::SLAB * sizeof(R);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (P.streaming)
-        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V>), dim3((unsigned)blocks),
+        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>), dim3((unsigned)blocks),
                            dim3(64 * wpb), lds, st, P);
     else
-        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V>), dim3((unsigned)blocks),
+        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>), dim3((unsigned)blocks),
                            dim3(64 * wpb), lds, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

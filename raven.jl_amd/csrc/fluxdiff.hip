@@ -450,9 +450,9 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
             }
             return TP::node(law, val);
         };
-        // FP32 state reads the FP32 copies of the 3-D geometry (every use
+        // FP32 state reads the FP32 copies of the geometry (every use
         // rounds to the state's type)
-        constexpr bool G32 = GEN && DIM == 3 && sizeof(R) == 4;
+        constexpr bool G32 = GEN && DIM > 1 && sizeof(R) == 4;
         using GT = typename std::conditional<G32, float, double>::type;
         const GT RV_GLOBAL *vgeo, *sgeo;
         if constexpr (G32)
@@ -719,7 +719,9 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
                 for (int s = 0; s < NS; ++s)
                     dqo[it][s] = load_dq<ST>(dq + off + s * NP);
             }
-            mji[it] = GEN ? R(P.mji[e * NP + node]) : R(1);
+            mji[it] = GEN && sizeof(R) == 4 ? R(P.mji32[e * NP + node])
+                      : GEN                 ? R(P.mji[e * NP + node])
+                                            : R(1);
             mj[it] = RX ? P.mj[e * NP + node] : 0.0;
         }
     }
@@ -811,7 +813,7 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
     R *qo = static_cast<R *>(P.q_out);
     const int64_t off = e * (NS * NP) + node;
     const int ijk[3] = {node % NQ, DIM > 1 ? (node / NQ) % NQ : 0, DIM > 2 ? node / (NQ * NQ) : 0};
-    constexpr bool G32 = GEN && DIM == 3 && sizeof(R) == 4;
+    constexpr bool G32 = GEN && DIM > 1 && sizeof(R) == 4;
     using GT = typename std::conditional<G32, float, double>::type;
     const GT RV_GLOBAL *vgeo, *sgeo;
     if constexpr (G32)
@@ -848,7 +850,7 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
                 dqo[s] = load_dq<ST>(dq + off + s * NP);
         }
         if constexpr (GEN)
-            mji = R(P.mji[e * NP + node]);
+            mji = G32 ? R(P.mji32[e * NP + node]) : R(P.mji[e * NP + node]);
         if constexpr (RX)
             mj = P.mj[e * NP + node];
         TP::values(law, q, x);

@@ -2,8 +2,8 @@
 // law) triple; the Makefile compiles this file once per triple with
 //   -DINST_DIM=<1|2|3> -DINST_REAL=<double|float> -DINST_LAW=<1|2> -DINST_FN=<name>
 // and api.hip asks every unit for a launcher.  3-D uses the column kernel
-// (dg_plane3.hpp), 2-D affine cells the node kernel (dg_quad2.hpp), 1-D and
-// 2-D general cells the pencil kernel (dg_kernels.hpp).
+// (dg_plane3.hpp), 2-D the node kernel (dg_quad2.hpp), 1-D the kernel of
+// dg_kernels.hpp.
 #include "dg_plane3.hpp"
 #include "dg_quad2.hpp"
 
@@ -26,8 +26,8 @@ StageLauncher pick_one(bool relax)
     } else {
         if (relax)
             return nullptr;  // the fused relaxation stage is built for 3-D
-        if constexpr (DIM == 2 && GEO == GEO_AFFINE)
-            return &launch_quad2<NQ, LAW, R, FLUX>;
+        if constexpr (DIM == 2)
+            return &launch_quad2<NQ, LAW, R, FLUX, GEO>;
         else
             return &launch_stage<DIM, NQ, LAW, R, GEO, FLUX>;
     }
