@@ -1,4 +1,5 @@
-// Fused DGSEM stage kernel for gfx950 (CDNA4, wave64).
+// The laws, fluxes and face indexing shared by the stage kernels, and the
+// fused 1-D DGSEM stage kernel for gfx950 (CDNA4, wave64).
 //
 // One fused launch computes, for every cell, Raven's weak-form volume term
 // (dgsem.jl:257-348), its surface term with the Rusanov/central flux
@@ -6,20 +7,10 @@
 // (odesolvers.jl:55-57):
 //     dq = a*dq + L(q_in);   q_out = q_in + b_dt*dq
 //
-// Work decomposition ("pencil sweeps").  A wave owns EPW = 64 / Nq^(dim-1)
-// cells; a lane owns one pencil (a line of Nq nodes) of one cell.  For each
-// direction d the lane loads its pencil along d, evaluates the flux component
-// needed by d, applies the 1-D derivative in registers (D is wave-uniform and
-// comes through scalar loads), and adds the lift of the two faces the pencil
-// ends on (faces 2d and 2d+1: their face node index equals the pencil index).
-// The directions' contributions meet in LDS (one slab per cell); the last
-// sweep adds them, applies the RK update and stores with lane-contiguous
-// addresses.  Neighbour states are read through per-face records (neighbour
-// cell, face, orientation), so a face costs 8 bytes of index traffic instead of
-// Nq^(dim-1) 8-byte node indices.
-//
-// Owner-computes: each cell evaluates the numerical flux of all of its faces;
-// no atomics, deterministic results.
+// Neighbour states are read through per-face records (neighbour cell, face,
+// orientation), so a face costs 8 bytes of index traffic instead of
+// Nq^(dim-1) 8-byte node indices.  Owner-computes: each cell evaluates the
+// numerical flux of all of its faces; no atomics, deterministic results.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -116,23 +107,6 @@ __device__ __host__ inline int orient_node(int o, int m)
         if (o & 2)
             b = NQ - 1 - b;
         return a + NQ * b;
-    }
-}
-
-template <int DIM, int NQ, int D>
-__device__ inline int pencil_base(int pen)
-{
-    if constexpr (DIM == 1) {
-        return 0;
-    } else if constexpr (DIM == 2) {
-        return D == 0 ? NQ * pen : pen;
-    } else {
-        if constexpr (D == 0)
-            return NQ * pen;
-        else if constexpr (D == 1)
-            return (pen % NQ) + NQ * NQ * (pen / NQ);
-        else
-            return pen;
     }
 }
 
@@ -250,7 +224,7 @@ struct Law {
 };
 
 // --------------------------------------------------------------------------
-// The kernel.
+// Numerical fluxes, and the 1-D kernel.
 // --------------------------------------------------------------------------
 
 // Loads and stores of a cell's own dq and q_out: plain (ST = 0), or streaming
@@ -350,224 +324,124 @@ struct Stage {
                 nf[s] = nf[s] - (lam * (qp[s] - qm[s])) * R(0.5);
         }
     }
+};
 
-    // One direction sweep; directions meet in the cell's LDS slab.  ST
-    // selects streaming accesses for dq and q_out (load_dq / store_out).
-    template <int D, int ST>
-    __device__ static inline void sweep(const StageParams &P, const Law<DIM, LAW, R> &law,
-                                        bool active, int64_t e, int pen, R *slab)
-    {
-        constexpr int STRIDE = IPow<NQ, D>::v;
-        constexpr bool FIRST = (D == 0);
-        constexpr bool LAST = (D == DIM - 1);
-        const int base = pencil_base<DIM, NQ, D>(pen);
-        const R *qbase = static_cast<const R *>(P.q_in);
-        const bool on = active && ((P.dir_mask >> D) & 1);
-
-        R F[NS][NQ];     // flux entering the derivative (contravariant for GENERAL)
-        R nf[2][NS];     // numerical flux at the two face nodes
-        R liftw[2];      // lift weight of the two face nodes
-        R scale = R(1);  // AFFINE: dRdX[D,D] of the cell
-
-        if (on) {
-            const R *qe = qbase + e * (NS * NP) + base;
-            R qv[NS][NQ];
+// The 1-D cells [cell0, cell0 + 64 / Nq) of a wave, a lane per node: states
+// with lane-contiguous addresses, the fluxes of a cell exchanged through the
+// wave's LDS row, the numerical flux of a face on the cell's end lanes.  A 1-D
+// stage is a few waves: it waits for one wave's chain of loads and the launch.
+template <int NQ, int LAW, typename R, int GEO, int FLUX, int ST>
+__device__ __attribute__((always_inline)) inline void stage_wave_1d(const StageParams &P,
+                                                                    int64_t cell0, R *wlds)
+{
+    using S = Stage<1, NQ, LAW, R, GEO, FLUX>;
+    constexpr int NS = S::NS, C = 64 / NQ;
+    constexpr bool GEN = GEO == GEO_GENERAL;
+    const int lane = threadIdx.x & 63;
+    const int c = lane / NQ, i = lane - c * NQ;
+    const int64_t e = cell0 + c;
+    const Law<1, LAW, R> law(P);
+    if (c < C && e < P.K) {
+        const bool on = P.dir_mask & 1;
+        const int side = i == NQ - 1;
+        const bool face = on && (i == 0 || side);
+        const int64_t off = e * (NS * NQ) + i;
+        const R *qin = static_cast<const R *>(P.q_in);
+        R *dq = static_cast<R *>(P.dq) + off;
+        R *qo = static_cast<R *>(P.q_out) + off;
+        R q[NS], qp[NS], dqo[NS], m[NQ], g = R(1), mji = R(1), nv[1] = {side ? R(1) : R(-1)}, lift;
 #pragma unroll
-            for (int n = 0; n < NQ; ++n)
+        for (int s = 0; s < NS; ++s)
+            q[s] = qin[off + s * NQ];
+        if (P.read_dq) {
 #pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    qv[s][n] = qe[s * NP + n * STRIDE];
-            // neighbour states first: their latency hides behind the flux work
-            R qp[2][NS];
-#pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                R qm[NS];
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    qm[s] = qv[s][side ? NQ - 1 : 0];
-                neighbour_state(P, qbase, e, 2 * D + side, pen, qm, qp[side]);
-            }
-#pragma unroll
-            for (int n = 0; n < NQ; ++n) {
-                R qn[NS];
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    qn[s] = qv[s][n];
-                if constexpr (GEO == GEO_AFFINE) {
-                    R f[NS];
-                    law.flux_row(D, qn, f);
-#pragma unroll
-                    for (int s = 0; s < NS; ++s)
-                        F[s][n] = f[s];
-                } else {
-                    R Fa[DIM][NS];
-                    law.flux_all(qn, Fa);
-                    const double *g = P.vgeo + ((e * DIM + D) * DIM) * NP + base + n * STRIDE;
-                    R gc[DIM];
-#pragma unroll
-                    for (int c = 0; c < DIM; ++c)
-                        gc[c] = R(g[c * NP]);
-#pragma unroll
-                    for (int s = 0; s < NS; ++s) {
-                        R v = gc[0] * Fa[0][s];
-#pragma unroll
-                        for (int c = 1; c < DIM; ++c)
-                            v = v + gc[c] * Fa[c][s];
-                        F[s][n] = v;
-                    }
-                }
-            }
-#pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                const int iend = side ? NQ - 1 : 0;
-                R qm[NS];
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    qm[s] = qv[s][iend];
-                if constexpr (GEO == GEO_AFFINE) {
-                    R fm[NS];
-#pragma unroll
-                    for (int s = 0; s < NS; ++s)
-                        fm[s] = F[s][iend];
-                    nflux_axis(law, D, side ? R(1) : R(-1), fm, qm, qp[side], nf[side]);
-                    liftw[side] = R(P.winv[iend]);
-                } else {
-                    const double *sg = P.sgeo + ((e * NF + 2 * D + side) * (DIM + 1)) * NP2 + pen;
-                    R nv[DIM];
-#pragma unroll
-                    for (int c = 0; c < DIM; ++c)
-                        nv[c] = R(sg[c * NP2]);
-                    liftw[side] = R(sg[DIM * NP2]);
-                    nflux_general(law, nv, qm, qp[side], nf[side]);
-                }
-            }
-            if constexpr (GEO == GEO_AFFINE)
-                scale = R(P.affine[e * DIM + D]);
+            for (int s = 0; s < NS; ++s)
+                dqo[s] = load_dq<ST>(dq + s * NQ);
         }
-
-        // state by state: derivative, lift, combine
-        const double *M = (GEO == GEO_AFFINE) ? P.Dw : P.Dt;
-        R *dq = static_cast<R *>(P.dq) + e * (NS * NP) + base;
-        const R *qe = qbase + e * (NS * NP) + base;
-        R *qo = static_cast<R *>(P.q_out) + e * (NS * NP) + base;
+        const double *M = GEN ? P.Dt : P.Dw;
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+            m[n] = R(M[i * NQ + n]);
+        if constexpr (GEN) {
+            g = R(P.vgeo[e * NQ + i]);
+            mji = R(P.mji[e * NQ + i]);
+        } else {
+            mji = R(P.affine[e]);
+        }
+        if (face) {
+            S::neighbour_state(P, qin, e, side, 0, q, qp);
+            if constexpr (GEN) {
+                nv[0] = R(P.sgeo[(e * 2 + side) * 2]);
+                lift = R(P.sgeo[(e * 2 + side) * 2 + 1]);
+            } else {
+                lift = R(P.winv[i]);
+            }
+        }
+        R f[NS];
+        law.flux_row(0, q, f);
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            wlds[s * 64 + lane] = g * f[s];
+        R nf[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            nf[s] = R(0);
+        if (face) {
+            if constexpr (GEN)
+                S::nflux_general(law, nv, q, qp, nf);
+            else
+                S::nflux_axis(law, 0, nv[0], f, q, qp, nf);
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                nf[s] = lift * nf[s];
+        }
+        wave_lds_sync();
         const R a = R(P.a), bdt = R(P.b_dt);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            R acc[NQ];
-#pragma unroll
-            for (int i = 0; i < NQ; ++i)
-                acc[i] = R(0);
+            R v = R(0);
             if (on) {
+                const R *row = wlds + s * 64 + lane - i;
+                v = m[0] * row[0];
 #pragma unroll
-                for (int i = 0; i < NQ; ++i) {
-                    R v = R(M[i * NQ]) * F[s][0];
-#pragma unroll
-                    for (int n = 1; n < NQ; ++n)
-                        v = v + R(M[i * NQ + n]) * F[s][n];
-                    acc[i] = v;
-                }
-                acc[0] = acc[0] - liftw[0] * nf[0][s];
-                acc[NQ - 1] = acc[NQ - 1] - liftw[1] * nf[1][s];
-                if constexpr (GEO == GEO_AFFINE) {
-#pragma unroll
-                    for (int i = 0; i < NQ; ++i)
-                        acc[i] = scale * acc[i];
-                }
+                for (int n = 1; n < NQ; ++n)
+                    v = v + m[n] * row[n];
+                v = mji * (v - nf[s]);
             }
-            if (!active)
-                continue;
-            if constexpr (!LAST) {
-#pragma unroll
-                for (int n = 0; n < NQ; ++n) {
-                    R *dst = slab + s * NP + base + n * STRIDE;
-                    if constexpr (FIRST)
-                        *dst = acc[n];
-                    else
-                        *dst = *dst + acc[n];
-                }
-            } else {
-#pragma unroll
-                for (int n = 0; n < NQ; ++n) {
-                    R tot = acc[n];
-                    if constexpr (DIM > 1)
-                        tot = slab[s * NP + base + n * STRIDE] + tot;
-                    if constexpr (GEO == GEO_GENERAL)
-                        tot = R(P.mji[e * NP + base + n * STRIDE]) * tot;
-                    // dq and q_out belong to this cell alone: on operators
-                    // larger than the caches they are streamed, which keeps
-                    // L2 for the shared q lines
-                    R v = tot;
-                    if (P.read_dq)
-                        v = a * load_dq<ST>(dq + s * NP + n * STRIDE) + tot;
-                    store_out<ST>(v, dq + s * NP + n * STRIDE);
-                    if (P.write_q)
-                        store_out<ST>(R(qe[s * NP + n * STRIDE] + bdt * v), qo + s * NP + n * STRIDE);
-                }
-            }
+            if (P.read_dq)
+                v = a * dqo[s] + v;
+            store_out<ST>(v, dq + s * NQ);
+            if (P.write_q)
+                store_out<ST>(R(q[s] + bdt * v), qo + s * NQ);
         }
-    }
-};
-
-// The cells [cell0, cell0 + EPW) of one wave (cell0 is the same on every
-// lane): the direction sweeps meet in the wave's own LDS slabs `wlds`
-// (EPW * Ns * Np values).
-template <int DIM, int NQ, int LAW, typename R, int GEO, int FLUX, int ST = 0>
-__device__ __attribute__((always_inline)) inline void stage_wave(const StageParams &P, int64_t cell0, R *wlds)
-{
-    using S = Stage<DIM, NQ, LAW, R, GEO, FLUX>;
-    constexpr int SLAB = S::NS * S::NP;
-    const int lane = threadIdx.x & 63;
-    const int slot = lane / S::NP2;
-    const int pen = lane - slot * S::NP2;
-    const int64_t e = cell0 + slot;
-    const bool active = (slot < S::EPW) && (e < P.K);
-    R *slab = wlds + (slot < S::EPW ? slot : 0) * SLAB;
-    const Law<DIM, LAW, R> law(P);
-
-    S::template sweep<0, ST>(P, law, active, e, pen, slab);
-    if constexpr (DIM > 1) {
-        wave_lds_sync();
-        S::template sweep<1, ST>(P, law, active, e, pen, slab);
-    }
-    if constexpr (DIM > 2) {
-        wave_lds_sync();
-        S::template sweep<2, ST>(P, law, active, e, pen, slab);
     }
 }
 
-// Waves per block (cells of one block share nothing; the knob trades LDS
-// granularity against scheduling) come from blockDim.x; the LDS slabs are
-// dynamic shared memory sized by the launcher.
-template <int DIM, int NQ, int LAW, typename R, int GEO, int FLUX, int ST>
-__global__ void __launch_bounds__(256) dg_stage_kernel(const StageParams P)
+// Waves per block come from blockDim.x; each has its own LDS rows.
+template <int NQ, int LAW, typename R, int GEO, int FLUX, int ST>
+__global__ void __launch_bounds__(256) dg_stage_kernel_1d(const StageParams P)
 {
-    using S = Stage<DIM, NQ, LAW, R, GEO, FLUX>;
-    extern __shared__ __attribute__((aligned(16))) unsigned char dg_lds[];
+    __shared__ R lds[4][LawInfo<1, LAW>::NS * 64];
     const int wave = threadIdx.x >> 6;
     const int wpb = blockDim.x >> 6;
     const int64_t blk = xcd_remap(blockIdx.x, gridDim.x);
-    const int64_t cell0 = (blk * wpb + wave) * S::EPW;
-    R *wlds = reinterpret_cast<R *>(dg_lds) + wave * S::EPW * S::NS * S::NP;
-    stage_wave<DIM, NQ, LAW, R, GEO, FLUX, ST>(P, cell0, wlds);
+    stage_wave_1d<NQ, LAW, R, GEO, FLUX, ST>(P, (blk * wpb + wave) * (64 / NQ), lds[wave]);
 }
 
-template <int DIM, int NQ, int LAW, typename R, int GEO, int FLUX>
-int launch_stage(const StageParams &P, void *stream, int wpb)
+template <int NQ, int LAW, typename R, int GEO, int FLUX>
+int launch_stage_1d(const StageParams &P, void *stream, int wpb)
 {
-    using S = Stage<DIM, NQ, LAW, R, GEO, FLUX>;
     if (P.K <= 0)
         return 0;
     if (wpb != 1 && wpb != 2 && wpb != 4)
         wpb = 1;
-    const int64_t waves = (P.K + S::EPW - 1) / S::EPW;
-    const int64_t blocks = (waves + wpb - 1) / wpb;
-    const size_t lds = DIM > 1 ? (size_t)wpb * S::EPW * S::NS * S::NP * sizeof(R) : 16;
+    const int64_t cells = (int64_t)wpb * (64 / NQ);
+    const dim3 grid((unsigned)((P.K + cells - 1) / cells)), block(64 * wpb);
+    hipStream_t st = static_cast<hipStream_t>(stream);
     if (P.streaming)
-        hipLaunchKernelGGL((dg_stage_kernel<DIM, NQ, LAW, R, GEO, FLUX, 1>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, static_cast<hipStream_t>(stream), P);
+        hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 1>), grid, block, 0, st, P);
     else
-        hipLaunchKernelGGL((dg_stage_kernel<DIM, NQ, LAW, R, GEO, FLUX, 0>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, static_cast<hipStream_t>(stream), P);
+        hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 0>), grid, block, 0, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

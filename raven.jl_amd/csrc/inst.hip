@@ -29,7 +29,7 @@ StageLauncher pick_one(bool relax)
         if constexpr (DIM == 2)
             return &launch_quad2<NQ, LAW, R, FLUX, GEO>;
         else
-            return &launch_stage<DIM, NQ, LAW, R, GEO, FLUX>;
+            return &launch_stage_1d<NQ, LAW, R, GEO, FLUX>;
     }
 }
 
