@@ -10,6 +10,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ravenhip.h"
@@ -88,8 +89,10 @@ struct rv_handle {
     double *relax_sums_host = nullptr;  // pinned copy of them
     double *eprod = nullptr;           // fused relaxation stages: 14 slots of relax_partials_cap
     void *qtmp = nullptr;        // ping-pong state of rv_lsrk_run
-    int64_t *dtoc = nullptr;     // 0-based
-    int64_t *ctod_ptr = nullptr;
+    // GatherScatter: indexes of 32 bits where the nodes allow it (wide: 64)
+    bool gs_wide = false;
+    char *dtoc = nullptr;        // 0-based
+    char *ctod_ptr = nullptr;
     int32_t *ctod_rows = nullptr;  // (cell, node) pairs
     int64_t nc = 0;
     int64_t device_bytes = 0;
@@ -258,80 +261,212 @@ __host__ __device__ inline double max_nan(double a, double b)
     return a != a ? a : b != b ? b : (a > b ? a : b);
 }
 
-// partial[s * RED_BLOCKS + block] = compensated sum over the block's share of
-// MJ * f(q_s); f = square (power 2), identity (power 1) or |q|^p (power 3);
-// power 4: the block's max |q_s| (in the sum slot, compensation 0)
-template <typename R>
+// partial[2 * (s * blocks + block)] = compensated sum over the block's share of
+// MJ * f(q_s) for every state s; f = square (MODE 2), identity (1) or |q|^p (3);
+// MODE 4: the block's max |q_s| (in the sum slot, compensation 0).  One sweep
+// over the nodes, all states of a node together: MJ crosses HBM once, no
+// division per node, four nodes' loads in flight per thread (2.28 M nodes,
+// five FP64 states: 23 us, 4.7 TB/s; a sweep per state with a 64-bit division
+// per element took 31 us).
+template <typename R, int NS, int MODE>
 __global__ void __launch_bounds__(RED_THREADS)
-    reduce_kernel(const R *q, const double *MJ, int64_t Np, int ns, int64_t K, int power,
-                  double pexp, double *partial)
+    reduce_kernel(const R *__restrict__ q, const double *__restrict__ MJ, int64_t Np, int64_t K,
+                  double pexp, double *__restrict__ partial)
 {
+    constexpr int U = 4;
     __shared__ Comp sh[RED_THREADS];
     const int64_t n = Np * K;
-    const int s = blockIdx.y;
-    Comp acc{0.0, 0.0};
+    Comp acc[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+        acc[s] = Comp{0.0, 0.0};
     const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
     const int64_t lo = (int64_t)blockIdx.x * chunk;
     const int64_t hi = (lo + chunk < n) ? lo + chunk : n;
-    for (int64_t i = lo + threadIdx.x; i < hi; i += RED_THREADS) {
-        const int64_t e = i / Np, node = i - e * Np;
-        const double v = (double)q[node + Np * (s + (int64_t)ns * e)];
-        if (power == 4) {
-            acc.s = max_nan(acc.s, fabs(v));
-            continue;
+    int64_t i = lo + threadIdx.x;
+    // the node's cell and place in it, stepped along with i
+    int64_t e = i / Np;
+    int node = (int)(i - e * Np);
+    const int de = (int)(RED_THREADS / Np), dn = (int)(RED_THREADS - de * Np);
+    while (i < hi) {
+        R v[U][NS];
+        double mj[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i + u * RED_THREADS < hi) {
+                const R *qe = q + e * (NS * Np) + node;
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    v[u][s] = qe[s * Np];
+                if constexpr (MODE != 4)
+                    mj[u] = MJ[i + u * RED_THREADS];
+            }
+            e += de;
+            node += dn;
+            if (node >= Np) {
+                node -= (int)Np;
+                ++e;
+            }
         }
-        const double x = power == 2   ? MJ[i] * (v * v)
-                         : power == 3 ? MJ[i] * pow(fabs(v), pexp)
-                                      : MJ[i] * v;
-        acc = comp_add(acc, x);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i + u * RED_THREADS < hi) {
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const double x = (double)v[u][s];
+                    if constexpr (MODE == 4)
+                        acc[s].s = max_nan(acc[s].s, fabs(x));
+                    else
+                        acc[s] = comp_add(acc[s], MODE == 2   ? mj[u] * (x * x)
+                                                  : MODE == 3 ? mj[u] * pow(fabs(x), pexp)
+                                                              : mj[u] * x);
+                }
+            }
+        i += U * RED_THREADS;
     }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            if (power == 4)
-                sh[threadIdx.x].s = max_nan(sh[threadIdx.x].s, sh[threadIdx.x + w].s);
-            else
-                sh[threadIdx.x] = comp_merge(sh[threadIdx.x], sh[threadIdx.x + w]);
-        }
+    for (int s = 0; s < NS; ++s) {
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        partial[2 * (s * RED_BLOCKS + blockIdx.x)] = sh[0].s;
-        partial[2 * (s * RED_BLOCKS + blockIdx.x) + 1] = sh[0].c;
+        sh[threadIdx.x] = acc[s];
+        __syncthreads();
+        for (int w = RED_THREADS / 2; w > 0; w >>= 1) {
+            if ((int)threadIdx.x < w) {
+                if constexpr (MODE == 4)
+                    sh[threadIdx.x].s = max_nan(sh[threadIdx.x].s, sh[threadIdx.x + w].s);
+                else
+                    sh[threadIdx.x] = comp_merge(sh[threadIdx.x], sh[threadIdx.x + w]);
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            partial[2 * (s * gridDim.x + blockIdx.x)] = sh[0].s;
+            partial[2 * (s * gridDim.x + blockIdx.x) + 1] = sh[0].c;
+        }
     }
 }
 
-// GatherScatter: dest[c + nc*s] = 0.0 + src[rows...] in ascending row order
-template <typename R>
-__global__ void gather_kernel(R *dest, const R *src, const int64_t *ptr, const int32_t *rows,
-                              int64_t nc, int64_t Np, int nf)
+template <typename R, int NS>
+void launch_reduce(const void *q, const double *MJ, int64_t Np, int64_t K, int mode, double pexp,
+                   double *partial, int blocks, hipStream_t st)
+{
+    const dim3 grid(blocks), block(RED_THREADS);
+    const R *p = static_cast<const R *>(q);
+    if (mode == 1)
+        hipLaunchKernelGGL((reduce_kernel<R, NS, 1>), grid, block, 0, st, p, MJ, Np, K, pexp, partial);
+    else if (mode == 2)
+        hipLaunchKernelGGL((reduce_kernel<R, NS, 2>), grid, block, 0, st, p, MJ, Np, K, pexp, partial);
+    else if (mode == 3)
+        hipLaunchKernelGGL((reduce_kernel<R, NS, 3>), grid, block, 0, st, p, MJ, Np, K, pexp, partial);
+    else
+        hipLaunchKernelGGL((reduce_kernel<R, NS, 4>), grid, block, 0, st, p, MJ, Np, K, pexp, partial);
+}
+
+// GatherScatter: dest[c + nc*s] = 0.0 + src[rows...] in ascending row order, a
+// thread per continuous node.  Up to eight rows (every conforming node has at
+// most 2^dim) are read first and then, field by field, their values, all in
+// flight before they are added in order: the kernel waits for scattered reads
+// (2.28 M nodes, five FP64 fields: 49 us, one read after another 86 us).
+// NF: the number of fields, 0 if not known here.
+template <typename R, typename I, int NF>
+__global__ void __launch_bounds__(256)
+    gather_kernel(R *__restrict__ dest, const R *__restrict__ src, const I *__restrict__ ptr,
+                  const int2 *__restrict__ rows, int64_t nc, int64_t Np, int nf_)
 {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nc)
         return;
-    const int64_t lo = ptr[c], hi = ptr[c + 1];
-    for (int s = 0; s < nf; ++s) {
-        R v = R(0);
-        for (int64_t r = lo; r < hi; ++r) {
-            const int64_t e = rows[2 * r], node = rows[2 * r + 1];
-            v = v + src[node + Np * (s + (int64_t)nf * e)];
+    const int nf = NF ? NF : nf_;
+    const int64_t lo = ptr[c];
+    const int n = (int)(ptr[c + 1] - lo);
+    constexpr int MOST = 8;
+    int64_t off[MOST];
+#pragma unroll
+    for (int k = 0; k < MOST; ++k)
+        if (k < n) {
+            const int2 r = rows[lo + k];
+            off[k] = r.y + Np * nf * r.x;
+        }
+    auto field = [&](int s) {
+        R x[MOST], v = R(0);
+#pragma unroll
+        for (int k = 0; k < MOST; ++k)
+            if (k < n)
+                x[k] = src[off[k] + Np * s];
+#pragma unroll
+        for (int k = 0; k < MOST; ++k)
+            if (k < n)
+                v = v + x[k];
+        for (int k = MOST; k < n; ++k) {
+            const int2 r = rows[lo + k];
+            v = v + src[r.y + Np * (s + (int64_t)nf * r.x)];
         }
         dest[c + nc * s] = v;
+    };
+    if constexpr (NF > 0) {
+#pragma unroll
+        for (int s = 0; s < NF; ++s)
+            field(s);
+    } else {
+        for (int s = 0; s < nf; ++s)
+            field(s);
     }
 }
 
-template <typename R>
-__global__ void scatter_kernel(R *dest, const R *src, const int64_t *dtoc, int64_t nc,
-                               int64_t Np, int64_t K, int nf)
+template <typename R, typename I, int NF>
+__global__ void __launch_bounds__(256)
+    scatter_kernel(R *__restrict__ dest, const R *__restrict__ src, const I *__restrict__ dtoc,
+                   int64_t nc, int64_t Np, int64_t K, int nf_)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= Np * K)
         return;
-    const int64_t e = i / Np, node = i - e * Np;
+    const int nf = NF ? NF : nf_;
+    // (node counts of 32-bit indexes divide in 32 bits)
+    const int64_t e = sizeof(I) == 4 ? (int64_t)((uint32_t)i / (uint32_t)Np) : i / Np;
+    const int64_t node = i - e * Np;
     const int64_t c = dtoc[i];
-    for (int s = 0; s < nf; ++s)
-        dest[node + Np * (s + (int64_t)nf * e)] = src[c + nc * s];
+    R *d = dest + node + Np * nf * e;
+    if constexpr (NF > 0) {
+        R x[NF];
+#pragma unroll
+        for (int s = 0; s < NF; ++s)
+            x[s] = src[c + nc * s];
+#pragma unroll
+        for (int s = 0; s < NF; ++s)
+            d[Np * s] = x[s];
+    } else {
+        for (int s = 0; s < nf; ++s)
+            d[Np * s] = src[c + nc * s];
+    }
+}
+
+template <typename R, typename I, int NF>
+void launch_gather_nf(bool scatter, void *dest, const void *src, const void *index,
+                      const int2 *rows, int64_t nc, int64_t Np, int64_t K, int nf, hipStream_t st)
+{
+    const int64_t n = scatter ? Np * K : nc;
+    const dim3 grid((unsigned)std::max<int64_t>((n + 255) / 256, 1)), block(256);
+    if (scatter)
+        hipLaunchKernelGGL((scatter_kernel<R, I, NF>), grid, block, 0, st, static_cast<R *>(dest),
+                           static_cast<const R *>(src), static_cast<const I *>(index), nc, Np, K,
+                           nf);
+    else
+        hipLaunchKernelGGL((gather_kernel<R, I, NF>), grid, block, 0, st, static_cast<R *>(dest),
+                           static_cast<const R *>(src), static_cast<const I *>(index), rows, nc,
+                           Np, nf);
+}
+
+// rv_gather / rv_scatter: one field and the states of the laws unrolled
+template <typename R, typename I>
+void launch_gather(bool scatter, void *dest, const void *src, const void *index, const int2 *rows,
+                   int64_t nc, int64_t Np, int64_t K, int nf, hipStream_t st)
+{
+    switch (nf) {
+    case 1: return launch_gather_nf<R, I, 1>(scatter, dest, src, index, rows, nc, Np, K, nf, st);
+    case 3: return launch_gather_nf<R, I, 3>(scatter, dest, src, index, rows, nc, Np, K, nf, st);
+    case 4: return launch_gather_nf<R, I, 4>(scatter, dest, src, index, rows, nc, Np, K, nf, st);
+    case 5: return launch_gather_nf<R, I, 5>(scatter, dest, src, index, rows, nc, Np, K, nf, st);
+    default: return launch_gather_nf<R, I, 0>(scatter, dest, src, index, rows, nc, Np, K, nf, st);
+    }
 }
 
 // Rebuild 1-based vmapM/vmapP/mapM/mapP from the face records.
@@ -618,7 +753,7 @@ int finish_setup(rv_handle *h, const double *D, const double *w)
     if ((rc = upload(h, &h->Dt, Dt.data(), Dt.size())) ||
         (rc = upload(h, &h->Dw, Dw.data(), Dw.size())) ||
         (rc = upload(h, &h->winv, winv.data(), winv.size())) ||
-        (rc = dalloc(h, &h->partials, (size_t)2 * RED_BLOCKS * h->ns)) ||
+        (rc = dalloc(h, &h->partials, (size_t)(2 * RED_BLOCKS + 1) * h->ns)) ||
         (rc = refresh_geo32(h)))
         return rc;
     if (h->vflux) {
@@ -686,9 +821,15 @@ int build_gatherscatter(rv_handle *h, const int64_t *dtoc, int64_t nc)
         rows[2 * r + 1] = (int32_t)(i % h->Np);
     }
     h->nc = nc;
+    h->gs_wide = n > INT32_MAX;
+    auto put = [&](char **dst, const std::vector<int64_t> &v) {
+        if (h->gs_wide)
+            return upload(h, dst, reinterpret_cast<const char *>(v.data()), v.size() * 8);
+        const std::vector<int32_t> w(v.begin(), v.end());
+        return upload(h, dst, reinterpret_cast<const char *>(w.data()), w.size() * 4);
+    };
     int rc;
-    if ((rc = upload(h, &h->dtoc, d0.data(), d0.size())) ||
-        (rc = upload(h, &h->ctod_ptr, ptr.data(), ptr.size())) ||
+    if ((rc = put(&h->dtoc, d0)) || (rc = put(&h->ctod_ptr, ptr)) ||
         (rc = upload(h, &h->ctod_rows, rows.data(), rows.size())))
         return rc;
     return RV_OK;
@@ -947,41 +1088,71 @@ int launch(rv_handle *h, const StageParams &P0, StageLauncher fn = nullptr)
     return RV_OK;
 }
 
-int reduce(rv_handle *h, const void *q, int power, double *out, double pexp = 2.0)
+// Sums over the states (reduce_kernel's modes) into out[ns], in a fixed order.
+// A block takes 2048 nodes or more; the partial sums of up to RED_HOST blocks
+// are added here, more of them on the device, where a second launch costs less
+// than the copy (40 cells of Nq = 5: 64 us for a norm, integrals, gather and
+// scatter with 512 blocks, 70 us with the second launch, 61 us so).
+constexpr int RED_HOST = 32;
+int reduce(rv_handle *h, const void *q, int mode, double *out, double pexp = 2.0)
 {
     if (!q)
         return fail(h, RV_E_ARG, "null state");
-    dim3 grid(RED_BLOCKS, h->ns);
-    if (h->dtype == RV_F64)
-        hipLaunchKernelGGL(reduce_kernel<double>, grid, dim3(RED_THREADS), 0, h->stream,
-                           static_cast<const double *>(q), h->MJ, h->Np, h->ns, h->K, power,
-                           pexp, h->partials);
-    else
-        hipLaunchKernelGGL(reduce_kernel<float>, grid, dim3(RED_THREADS), 0, h->stream,
-                           static_cast<const float *>(q), h->MJ, h->Np, h->ns, h->K, power,
-                           pexp, h->partials);
+    const int ns = h->ns;
+    const int blocks =
+        (int)std::min<int64_t>(RED_BLOCKS, std::max<int64_t>(1, h->Np * h->K / 2048));
+    auto run = [&](auto n) {
+        constexpr int NS = decltype(n)::value;
+        if (h->dtype == RV_F64)
+            launch_reduce<double, NS>(q, h->MJ, h->Np, h->K, mode, pexp, h->partials, blocks,
+                                      h->stream);
+        else
+            launch_reduce<float, NS>(q, h->MJ, h->Np, h->K, mode, pexp, h->partials, blocks,
+                                     h->stream);
+    };
+    switch (ns) {
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    case 4: run(std::integral_constant<int, 4>{}); break;
+    case 5: run(std::integral_constant<int, 5>{}); break;
+    default: return fail(h, RV_E_UNSUPPORTED, "reduction over this number of states");
+    }
     HIP_TRY(h, hipGetLastError());
-    std::vector<double> part((size_t)2 * RED_BLOCKS * h->ns);
-    HIP_TRY(h, hipMemcpyAsync(part.data(), h->partials, part.size() * sizeof(double),
+    double part[2 * RED_HOST * 5];
+    if (mode != 4 && blocks > RED_HOST) {
+        double *sums = h->partials + (size_t)2 * RED_BLOCKS * ns;
+        if (launch_slot_sums(h->partials, 2 * blocks, ns, 1, 2 * blocks, 0, 1, 1, sums,
+                             h->stream) != 0) {
+            hipError_t e = hipGetLastError();
+            return fail(h, RV_E_HIP,
+                        std::string("reduction launch failed: ") + hipGetErrorString(e));
+        }
+        HIP_TRY(h, hipMemcpyAsync(part, sums, ns * sizeof(double), hipMemcpyDeviceToHost,
+                                  h->stream));
+        HIP_TRY(h, hipStreamSynchronize(h->stream));
+        std::copy(part, part + ns, out);
+        return RV_OK;
+    }
+    std::vector<double> many(blocks > RED_HOST ? (size_t)2 * blocks * ns : 0);
+    double *p = blocks > RED_HOST ? many.data() : part;
+    HIP_TRY(h, hipMemcpyAsync(p, h->partials, (size_t)2 * blocks * ns * sizeof(double),
                               hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(h, hipStreamSynchronize(h->stream));
-    for (int s = 0; s < h->ns; ++s) {
-        if (power == 4) {
+    for (int s = 0; s < ns; ++s) {
+        if (mode == 4) {
             double m = 0.0;
-            for (int b = 0; b < RED_BLOCKS; ++b)
-                m = max_nan(m, part[2 * (s * RED_BLOCKS + b)]);
+            for (int b = 0; b < blocks; ++b)
+                m = max_nan(m, p[2 * (s * blocks + b)]);
             out[s] = m;
             continue;
         }
         // Neumaier over the block partials in block order
         double sum = 0, comp = 0;
-        for (int b = 0; b < RED_BLOCKS; ++b) {
-            for (int k = 0; k < 2; ++k) {
-                const double x = part[2 * (s * RED_BLOCKS + b) + k];
-                const double t = sum + x;
-                comp += std::fabs(sum) >= std::fabs(x) ? (sum - t) + x : (x - t) + sum;
-                sum = t;
-            }
+        for (int k = 0; k < 2 * blocks; ++k) {
+            const double x = p[2 * s * blocks + k];
+            const double t = sum + x;
+            comp += std::fabs(sum) >= std::fabs(x) ? (sum - t) + x : (x - t) + sum;
+            sum = t;
         }
         out[s] = sum + comp;
     }
@@ -1957,45 +2128,32 @@ int ensure_gatherscatter(rv_handle *h)
 }
 }  // namespace
 
-int rv_gather(rv_handle *h, void *dest, const void *src, int nf)
+static int gather_scatter(rv_handle *h, bool scatter, void *dest, const void *src, int nf)
 {
     if (!h || !dest || !src || nf < 1)
         return fail(h, RV_E_ARG, "invalid argument");
     if (int rc = ensure_gatherscatter(h))
         return rc;
-    const int64_t blocks = (h->nc + 255) / 256;
+    const void *index = scatter ? h->dtoc : h->ctod_ptr;
+    const int2 *rows = reinterpret_cast<const int2 *>(h->ctod_rows);
     if (h->dtype == RV_F64)
-        hipLaunchKernelGGL(gather_kernel<double>, dim3((unsigned)std::max<int64_t>(blocks, 1)),
-                           dim3(256), 0, h->stream, static_cast<double *>(dest),
-                           static_cast<const double *>(src), h->ctod_ptr, h->ctod_rows, h->nc,
-                           h->Np, nf);
+        (h->gs_wide ? launch_gather<double, int64_t> : launch_gather<double, int32_t>)(
+            scatter, dest, src, index, rows, h->nc, h->Np, h->K, nf, h->stream);
     else
-        hipLaunchKernelGGL(gather_kernel<float>, dim3((unsigned)std::max<int64_t>(blocks, 1)),
-                           dim3(256), 0, h->stream, static_cast<float *>(dest),
-                           static_cast<const float *>(src), h->ctod_ptr, h->ctod_rows, h->nc,
-                           h->Np, nf);
+        (h->gs_wide ? launch_gather<float, int64_t> : launch_gather<float, int32_t>)(
+            scatter, dest, src, index, rows, h->nc, h->Np, h->K, nf, h->stream);
     HIP_TRY(h, hipGetLastError());
     return RV_OK;
 }
 
+int rv_gather(rv_handle *h, void *dest, const void *src, int nf)
+{
+    return gather_scatter(h, false, dest, src, nf);
+}
+
 int rv_scatter(rv_handle *h, void *dest, const void *src, int nf)
 {
-    if (!h || !dest || !src || nf < 1)
-        return fail(h, RV_E_ARG, "invalid argument");
-    if (int rc = ensure_gatherscatter(h))
-        return rc;
-    const int64_t n = h->Np * h->K;
-    const int64_t blocks = std::max<int64_t>((n + 255) / 256, 1);
-    if (h->dtype == RV_F64)
-        hipLaunchKernelGGL(scatter_kernel<double>, dim3((unsigned)blocks), dim3(256), 0, h->stream,
-                           static_cast<double *>(dest), static_cast<const double *>(src), h->dtoc,
-                           h->nc, h->Np, h->K, nf);
-    else
-        hipLaunchKernelGGL(scatter_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, h->stream,
-                           static_cast<float *>(dest), static_cast<const float *>(src), h->dtoc,
-                           h->nc, h->Np, h->K, nf);
-    HIP_TRY(h, hipGetLastError());
-    return RV_OK;
+    return gather_scatter(h, true, dest, src, nf);
 }
 
 int rv_get_maps(rv_handle *h, int64_t *vmapM, int64_t *vmapP, int64_t *mapM, int64_t *mapP)
