@@ -1042,10 +1042,13 @@ StageParams stage_params(rv_handle *h)
     for (int c = 0; c < 3; ++c)
         P.u[c] = h->u[c];
     // a stage touches q_in, dq and q_out; beyond the 256 MB Infinity Cache of
-    // MI355X nothing of dq and q_out survives to the next stage, so they are
-    // streamed past L2 (which then keeps the q lines that face reads share)
-    const int64_t state = h->Np * h->ns * h->K * (h->dtype == RV_F32 ? 4 : 8);
-    P.streaming = 3 * state > STREAM_BYTES ? 1 : 0;
+    // MI355X nothing of dq and q_out survives to the next stage, so kernels
+    // that write whole lines (stage_streams) stream them past L2 (which then
+    // keeps the q lines that face reads share)
+    const int b = h->dtype == RV_F32 ? 4 : 8;
+    const int64_t state = h->Np * h->ns * h->K * b;
+    P.streaming =
+        3 * state > STREAM_BYTES && stage_streams(h->dim, h->nq, h->law, b, h->geo, h->vflux) ? 1 : 0;
     return P;
 }
 

@@ -91,6 +91,28 @@ struct StageParams {
     const void RV_GLOBAL *mdelta;
 };
 
+// Whether a stage larger than the caches streams dq and q_out past them
+// (StageParams::streaming).  A launch writes a cell's states in pieces: the
+// weak form Nq^2 values (2-D a cell, 3-D a plane), flux differencing a cell.
+// Streamed pieces that end inside a 128-byte line reach HBM as partial writes,
+// where the caches would have joined them; one state per cell (advection)
+// leaves no gaps between the cells.  us per Euler stage, streamed / not: 3-D Nq = 8
+// FP64 28^3 348 / 389, Nq = 4 FP64 46^3 196 / 242, but Nq = 5 FP64 44^3 594 /
+// 448, FP32 412 / 272, Nq = 7 FP32 32^3 316 / 256; 2-D Nq = 8 FP64 390^2 274 /
+// 286, Nq = 4 FP32 760^2 198 / 167, Nq = 5 FP64 620^2 356 / 318; entropy-
+// conservative form, 2-D Nq = 5 FP64 620^2 385 / 351, curved 3-D Nq = 5 FP32
+// 40^3 380 / 367.  On 3-D affine cells whole 32-byte sectors (Nq = 6 FP64 30^3
+// 227 / 241, 38^3 474 / 462; curved 394 / 377, 794 / 729), and for flux
+// differencing any cell (Nq = 5 FP64 40^3 376 / 402), are enough.
+constexpr bool stage_streams(int dim, int nq, int law, int real_bytes, int geo, int vflux)
+{
+    if (law == LAW_ADVECTION)
+        return true;
+    const bool brick3 = dim == 3 && geo == GEO_AFFINE;
+    const int piece = (dim == 1 ? nq : dim == 3 && vflux ? nq * nq * nq : nq * nq) * real_bytes;
+    return piece % (brick3 && vflux ? 1 : brick3 ? 32 : 128) == 0;
+}
+
 // Product slots (StageParams::eprod) the 3-D column kernel's relaxation stage
 // writes, one per wave launched: Nq = 5, 6, 7 pack 64 G / Nq^2 cells into a
 // workgroup of G = 2, 4, 4 waves, the others give a wave 64 / Nq^2 cells and a

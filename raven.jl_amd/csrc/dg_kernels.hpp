@@ -438,10 +438,14 @@ int launch_stage_1d(const StageParams &P, void *stream, int wpb)
     const int64_t cells = (int64_t)wpb * (64 / NQ);
     const dim3 grid((unsigned)((P.K + cells - 1) / cells)), block(64 * wpb);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (P.streaming)
-        hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 1>), grid, block, 0, st, P);
-    else
-        hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 0>), grid, block, 0, st, P);
+    if constexpr (stage_streams(1, NQ, LAW, sizeof(R), GEO, 0)) {
+        if (P.streaming) {
+            hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 1>), grid, block, 0, st,
+                               P);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
+    }
+    hipLaunchKernelGGL((dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 0>), grid, block, 0, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

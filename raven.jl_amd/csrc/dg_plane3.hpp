@@ -764,12 +764,16 @@ int launch_plane3_rx(const StageParams &P, void *stream, int wpb)
         blocks = (waves + wpb - 1) / wpb;
         lds = (size_t)wpb * T::EPW * T::SLAB * sizeof(R);
     }
-    if (P.streaming)
-        hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, static_cast<hipStream_t>(stream), P);
-    else
-        hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, static_cast<hipStream_t>(stream), P);
+    const dim3 grid((unsigned)blocks), block(64 * wpb);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if constexpr (stage_streams(3, NQ, LAW, sizeof(R), GEO, 0)) {
+        if (P.streaming) {
+            hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX>), grid, block, lds,
+                               st, P);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
+    }
+    hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX>), grid, block, lds, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -340,12 +340,15 @@ int launch_quad2(const StageParams &P, void *stream, int wpb)
     const int64_t blocks = (groups + gpb - 1) / gpb;
     const size_t lds = (size_t)gpb * Q::SLAB * sizeof(R);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (P.streaming)
-        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, st, P);
-    else
-        hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>), dim3((unsigned)blocks),
-                           dim3(64 * wpb), lds, st, P);
+    const dim3 grid((unsigned)blocks), block(64 * wpb);
+    if constexpr (stage_streams(2, NQ, LAW, sizeof(R), GEO, 0)) {
+        if (P.streaming) {
+            hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>), grid, block, lds,
+                               st, P);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
+    }
+    hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>), grid, block, lds, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

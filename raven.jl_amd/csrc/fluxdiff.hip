@@ -1058,10 +1058,13 @@ int launch_fd(const StageParams &P, void *stream, int)
     if (P.K <= 0)
         return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (P.streaming)
-        launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, st);
-    else
-        launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 0>(P, st);
+    if constexpr (stage_streams(DIM, NQ, LAW, sizeof(R), GEO, VF)) {
+        if (P.streaming) {
+            launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, st);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
+    }
+    launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 0>(P, st);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
