@@ -113,16 +113,47 @@ constexpr bool stage_streams(int dim, int nq, int law, int real_bytes, int geo, 
     return piece % (brick3 && vflux ? 1 : brick3 ? 32 : 128) == 0;
 }
 
+// Waves of a workgroup of the 3-D column kernel that packs its cells across
+// lanes (dg_plane3.hpp), 1: nothing to gain.
+constexpr int plane3_pack_waves(int nq) { return nq == 5 ? 2 : nq == 6 || nq == 7 ? 4 : 1; }
+
+// Whether a launch over K cells packs them.  Packing fills lanes but ties the
+// waves of a workgroup together: with one wave per cell and at most 1024 cells
+// of Nq = 6 or 2048 of Nq = 7 every cell is resident at once (one or two waves
+// per SIMD) and packing only lengthens each wave's chain; beyond the caches, where the waits
+// are longest, FP32 and curved cells gain from independent waves too, and
+// Nq = 7, whose cells leave few lanes idle, in every form but affine FP64 in
+// the caches.  us per Euler stage, packed / one wave per cell: 8^3 cells of
+// Nq = 6 FP64 16.4 / 13.0, 12^3 21.3 / 22.5, 20^3 72.1 / 78.8, 38^3 470 / 528, FP32 274 / 258, curved
+// FP32 404 / 393, FP64 729 / 789; 7^3 of Nq = 7 FP64 25.0 / 16.8, 12^3 43.7 / 37.8, 17^3 84.6 / 87.5,
+// FP32 42.7 / 39.9, curved FP64 146 / 140, 32^3 FP64 549 / 520, curved 921 / 802, FP32
+// 256 / 235; Nq = 5 10^3 FP64 12.1 / 14.1, 44^3 FP64 448 / 445, FP32 272 / 260, curved
+// FP32 408 / 385, FP64 717 / 698.
+inline bool plane3_packed(int nq, int law, int real_bytes, int geo, int64_t K)
+{
+    if (plane3_pack_waves(nq) == 1)
+        return false;
+    const int ns = law == LAW_ADVECTION ? 1 : 5;
+    const bool large = 3 * K * nq * nq * nq * ns * real_bytes > ((int64_t)256 << 20);
+    const bool curved = geo != GEO_AFFINE;
+    if (nq == 5)
+        return !(large && (real_bytes == 4 || curved));
+    if (K <= (nq == 6 ? 1024 : 2048))
+        return false;
+    if (nq == 6)
+        return !(large && real_bytes == 4);
+    return real_bytes == 8 && !curved && !large;
+}
+
 // Product slots (StageParams::eprod) the 3-D column kernel's relaxation stage
-// writes, one per wave launched: Nq = 5, 6, 7 pack 64 G / Nq^2 cells into a
-// workgroup of G = 2, 4, 4 waves, the others give a wave 64 / Nq^2 cells and a
-// workgroup wpb waves.
-inline int64_t plane3_relax_slots(int nq, int64_t K, int wpb)
+// writes, one per wave launched: a packed launch has 64 G / Nq^2 cells to a
+// workgroup of G waves, the others 64 / Nq^2 cells to a wave and wpb waves to a
+// workgroup.
+inline int64_t plane3_relax_slots(int nq, int law, int real_bytes, int geo, int64_t K, int wpb)
 {
     const int nq2 = nq * nq;
-    const int g = nq == 5 ? 2 : (nq == 6 || nq == 7) ? 4 : 1;
-    if (g > 1) {
-        const int cpg = 64 * g / nq2;
+    if (plane3_packed(nq, law, real_bytes, geo, K)) {
+        const int g = plane3_pack_waves(nq), cpg = 64 * g / nq2;
         return (K + cpg - 1) / cpg * g;
     }
     if (wpb != 1 && wpb != 2 && wpb != 4)

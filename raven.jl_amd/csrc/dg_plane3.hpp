@@ -81,12 +81,12 @@ struct Plane3 {
     static constexpr int CTAB = WLDS ? 2 * NQ2 : 0;
     static constexpr int SLAB = SLAB0 + XFB + CTAB;
     static_assert(EPW >= 1, "Nq^2 must not exceed the wave size");
-    // Waves that share their cells: Nq^2 of 25, 36 or 49 columns leave 14 to
-    // 44 % of a wave's lanes idle when cells do not straddle waves, so a
-    // workgroup of G waves packs CPG cells across its 64 G lanes instead
-    // (125 of 128, 252 of 256, 245 of 256 lanes busy) and synchronises its
-    // LDS slabs with workgroup barriers.
-    static constexpr int G = (NQ == 5) ? 2 : (NQ == 6 || NQ == 7) ? 4 : 1;
+    // Waves that share their cells in a packed launch (plane3_packed): Nq^2 of
+    // 25, 36 or 49 columns leave 14 to 44 % of a wave's lanes idle when cells
+    // do not straddle waves, so a workgroup of G waves packs CPG cells across
+    // its 64 G lanes (125 of 128, 252 of 256, 245 of 256 lanes busy) and
+    // synchronises its LDS slabs with workgroup barriers.
+    static constexpr int G = plane3_pack_waves(NQ);
     static constexpr int CPG = 64 * G / NQ2;
     using S = Stage<3, NQ, LAW, R, GEO, FLUX>;
 };
@@ -722,7 +722,7 @@ __device__ __attribute__((always_inline)) inline void plane3_wave(const StagePar
     }
 }
 
-template <int NQ, int LAW, typename R, int GEO, int FLUX, int ST, int RX = 0>
+template <int NQ, int LAW, typename R, int GEO, int FLUX, int ST, int RX, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 dg_plane3_kernel(const StageParams P)
 {
@@ -733,10 +733,10 @@ dg_plane3_kernel(const StageParams P)
     const int wpb = blockDim.x >> 6;
     // RX: one product slot per wave of the launch
     const int64_t eslot = blk * wpb + wave;
-    if constexpr (T::G > 1) {
+    if constexpr (G > 1) {
         // one workgroup of G waves packs CPG cells
-        plane3_wave<NQ, LAW, R, GEO, FLUX, ST, T::G, RX>(P, blk * T::CPG,
-                                                         reinterpret_cast<R *>(dg_lds), eslot);
+        plane3_wave<NQ, LAW, R, GEO, FLUX, ST, G, RX>(P, blk * T::CPG,
+                                                      reinterpret_cast<R *>(dg_lds), eslot);
     } else {
         R *wlds = reinterpret_cast<R *>(dg_lds) + wave * T::EPW * T::SLAB;
         plane3_wave<NQ, LAW, R, GEO, FLUX, ST, 1, RX>(P, (blk * wpb + wave) * T::EPW, wlds,
@@ -744,19 +744,17 @@ dg_plane3_kernel(const StageParams P)
     }
 }
 
-template <int NQ, int LAW, typename R, int GEO, int FLUX, int RX>
-int launch_plane3_rx(const StageParams &P, void *stream, int wpb)
+template <int NQ, int LAW, typename R, int GEO, int FLUX, int RX, int G>
+int launch_plane3_g(const StageParams &P, void *stream, int wpb)
 {
     using T = Plane3<NQ, LAW, R, GEO, FLUX>;
-    if (P.K <= 0)
-        return 0;
     if (wpb != 1 && wpb != 2 && wpb != 4)
         wpb = 1;
     int64_t blocks;
     size_t lds;
-    if constexpr (T::G > 1) {
+    if constexpr (G > 1) {
         // packed cells: the workgroup is the G waves that share them
-        wpb = T::G;
+        wpb = G;
         blocks = (P.K + T::CPG - 1) / T::CPG;
         lds = (size_t)T::CPG * T::SLAB * sizeof(R);
     } else {
@@ -768,13 +766,27 @@ int launch_plane3_rx(const StageParams &P, void *stream, int wpb)
     hipStream_t st = static_cast<hipStream_t>(stream);
     if constexpr (stage_streams(3, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
-            hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX>), grid, block, lds,
-                               st, P);
+            hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX, G>), grid, block,
+                               lds, st, P);
             return hipGetLastError() == hipSuccess ? 0 : -1;
         }
     }
-    hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX>), grid, block, lds, st, P);
+    hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX, G>), grid, block, lds, st,
+                       P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <int NQ, int LAW, typename R, int GEO, int FLUX, int RX>
+int launch_plane3_rx(const StageParams &P, void *stream, int wpb)
+{
+    constexpr int G = plane3_pack_waves(NQ);
+    if (P.K <= 0)
+        return 0;
+    if constexpr (G > 1) {
+        if (plane3_packed(NQ, LAW, sizeof(R), GEO, P.K))
+            return launch_plane3_g<NQ, LAW, R, GEO, FLUX, RX, G>(P, stream, wpb);
+    }
+    return launch_plane3_g<NQ, LAW, R, GEO, FLUX, RX, 1>(P, stream, wpb);
 }
 
 template <int NQ, int LAW, typename R, int GEO, int FLUX>
