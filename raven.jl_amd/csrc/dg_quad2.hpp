@@ -17,9 +17,9 @@
 //    share one workgroup's cells (5, 7, 5 cells over 128, 256, 256 lanes) and
 //    synchronise with workgroup barriers (so do batches launching a kind on
 //    its own); the batches' work-list kernel uses G = 1;
-//  * light cells (advection, FP32 Euler) give a lane V = 4 or 2 nodes, one in
-//    each of V sets of cells, all requested before the first wait: a wave
-//    then has V times the bytes in flight;
+//  * light cells (advection, FP32 Euler) of a grid that fills the device give
+//    a lane V = 4 or 2 nodes, one in each of V sets of cells, all requested
+//    before the first wait: a wave then has V times the bytes in flight;
 //  * curved cells publish contravariant fluxes and lifted numerical fluxes.
 //    Bound by memory: on 200^2 warped cells of Nq = 6 an FP64 Euler stage
 //    takes 41.5 us (6.0 TB/s, out of the Infinity Cache; a lane per pencil,
@@ -320,17 +320,11 @@ __global__ void __launch_bounds__(256) dg_quad2_kernel(const StageParams P)
     quad2_group<NQ, LAW, R, FLUX, ST, G, V, GEO>(P, (blk * gpb + grp) * Q::CELLS, glds, gl);
 }
 
-template <int NQ, int LAW, typename R, int FLUX, int GEO>
-int launch_quad2(const StageParams &P, void *stream, int wpb)
+template <int NQ, int LAW, typename R, int FLUX, int GEO, int V>
+int launch_quad2_v(const StageParams &P, void *stream, int wpb)
 {
     constexpr int G = quad2_group_waves<NQ>();
-    // (curved cells: one node per lane, whose metric terms are bytes enough in
-    // flight: 2 took 44 to 51 us against 41 to 46 us per FP64 Euler stage of
-    // 1.4 to 1.6 M nodes, advection likewise)
-    constexpr int V = GEO == GEO_GENERAL ? 1 : quad2_nodes_per_lane<LAW, R>();
     using Q = Quad2<NQ, LAW, R, FLUX, G, V>;
-    if (P.K <= 0)
-        return 0;
     if (G > 1)
         wpb = G;
     else if (wpb != 1 && wpb != 2 && wpb != 4)
@@ -350,6 +344,32 @@ int launch_quad2(const StageParams &P, void *stream, int wpb)
     }
     hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>), grid, block, lds, st, P);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <int NQ, int LAW, typename R, int FLUX, int GEO>
+int launch_quad2(const StageParams &P, void *stream, int wpb)
+{
+    constexpr int G = quad2_group_waves<NQ>();
+    // (curved cells: one node per lane, whose metric terms are bytes enough in
+    // flight: 2 took 44 to 51 us against 41 to 46 us per FP64 Euler stage of
+    // 1.4 to 1.6 M nodes, advection likewise)
+    constexpr int V = GEO == GEO_GENERAL ? 1 : quad2_nodes_per_lane<LAW, R>();
+    if (P.K <= 0)
+        return 0;
+    // A grid that leaves the device room for its waves is not bound by bytes
+    // but by one wave's pass through the code, fetched cold at each launch, and
+    // V nodes per lane make that V times as long: one node per lane up to 24
+    // waves per CU (256 CUs).  FP64 advection, us per LSRK stage, V nodes / one:
+    // Nq = 5 on 16^2 4.98 / 2.95, 96^2 (3687 waves) 5.81 / 4.78, 128^2 (6554)
+    // 6.86 / 6.32, 192^2 (14746) 9.94 / 11.0; Nq = 8 on 64^2 (4096) 5.64 / 5.10,
+    // 96^2 (9216) 7.77 / 8.81.  FP32 Euler, Nq = 5: 5.40 / 3.99 on 16^2, even
+    // from 96^2 on.
+    if constexpr (V > 1) {
+        constexpr int cells = 64 * G / (NQ * NQ);
+        if (!P.streaming && (P.K + cells - 1) / cells * G <= 6144)
+            return launch_quad2_v<NQ, LAW, R, FLUX, GEO, 1>(P, stream, wpb);
+    }
+    return launch_quad2_v<NQ, LAW, R, FLUX, GEO, V>(P, stream, wpb);
 }
 
 }  // namespace rv

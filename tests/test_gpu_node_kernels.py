@@ -81,3 +81,15 @@ def test_2d_warped_stage(torch, R, nq, law, dtype):
 
     for n in ([2, 1], [5, 3], [17, 7]):
         check_stage(torch, R, 2, nq, n, law, dtype, "auto", warp)
+
+
+@pytest.mark.parametrize("law,dtype", [("advection", "f64"), ("advection", "f32"),
+                                       ("euler", "f32")])
+@pytest.mark.parametrize("nq", range(2, 9))
+def test_2d_nodes_per_lane(torch, R, nq, law, dtype):
+    """Affine 2-D cells that give a lane several nodes on large grids: both
+    sides of the size where the launch changes over, and a remainder."""
+    waves = {5: 2, 6: 4, 7: 4}.get(nq, 1)  # sharing a group's cells
+    line = 64 * waves // nq**2 * (6144 // waves)
+    for K in (line, line + 1, line + 37):
+        check_stage(torch, R, 2, nq, [K, 1], law, dtype, "auto")
