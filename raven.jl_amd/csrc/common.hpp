@@ -42,7 +42,9 @@ inline T RV_GLOBAL *as_global(T *p)
     return (T RV_GLOBAL *)p;
 }
 
-// Arguments of one fused DG stage launch.  Pointers are device pointers.
+// Arguments of one fused DG stage launch.  Pointers are device pointers.  What the
+// affine weak form reads comes first, in two 64-byte lines of the (cold) scalar
+// cache.
 struct StageParams {
     int64_t K;            // cells
     const void RV_GLOBAL *q_in;  // state read (R)
@@ -50,14 +52,25 @@ struct StageParams {
     void RV_GLOBAL *dq;          // register (R)
     double a;             // dq = a*dq + L
     double b_dt;          // q_out = q_in + b_dt*dq
-    int read_dq;          // load dq (a != 0 or increment)
-    int write_q;          // stage mode
-    int dir_mask;         // active directions (bit d)
-    int streaming;        // dq and q_out through L2 as streaming (non-temporal) accesses
+    int16_t read_dq;      // load dq (a != 0 or increment)
+    int16_t write_q;      // stage mode
+    int16_t dir_mask;     // active directions (bit d)
+    int16_t streaming;    // dq and q_out through L2 as streaming (non-temporal) accesses
+    // the launch's own shape (launch_stage): workgroups and waves in each.  The
+    // kernels read it here, with the rest, and not through blockDim and gridDim,
+    // which the runtime puts behind the arguments: two more lines to fetch
+    uint32_t blocks;
+    int32_t wpb;
     const FaceRec RV_GLOBAL *faces;        // (2dim, K)
     const int64_t RV_GLOBAL *explicit_idx; // explicit face-node offsets
     // affine geometry: per cell, per direction: dRdX[d,d] (FP64)
     const double RV_GLOBAL *affine;        // (K, dim)
+    // operators (FP64, device)
+    const double RV_GLOBAL *Dw;    // [i*Nq + n] = D[n,i] w_n / w_i  (affine)
+    const double RV_GLOBAL *winv;  // [i] = 1/w_i
+    double gamma;
+    double u[3];
+    const double RV_GLOBAL *Dt;    // [i*Nq + n] = D[n,i]            (general)
     // general geometry (FP64): wJ*dRdX rows, MJI, face normals and wsJ
     const double RV_GLOBAL *vgeo;  // (K, dim, dim, Np): [e][d][c][node] = wJ*dRdX[d,c]
     const double RV_GLOBAL *mji;   // (K, Np)
@@ -70,15 +83,9 @@ struct StageParams {
     const float RV_GLOBAL *mji32;
     const float RV_GLOBAL *sgeo32;
     const float RV_GLOBAL *mj32;
-    // operators (FP64, device)
-    const double RV_GLOBAL *Dt;    // [i*Nq + n] = D[n,i]            (general)
-    const double RV_GLOBAL *Dw;    // [i*Nq + n] = D[n,i] w_n / w_i  (affine)
-    const double RV_GLOBAL *winv;  // [i] = 1/w_i
     // flux differencing, in the state's type: [i*Nq + n] = D[n,i] w_n / w_i - D[i,n]
     // (affine), then [i*Nq + n] = D[i,n] (general)
     const void RV_GLOBAL *fdtab;
-    double gamma;
-    double u[3];
     // relaxation stage (the flux-differencing kernels built for it): dq = a dq + k
     // with k = L(q_in) accumulated alone, and each workgroup stores
     // sum MJ v(q_in) . k over its nodes at eprod[workgroup]

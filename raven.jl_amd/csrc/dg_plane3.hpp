@@ -728,9 +728,9 @@ dg_plane3_kernel(const StageParams P)
 {
     using T = Plane3<NQ, LAW, R, GEO, FLUX>;
     extern __shared__ __attribute__((aligned(16))) unsigned char dg_lds[];
-    const int64_t blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t blk = xcd_remap(blockIdx.x, P.blocks);
     const int wave = threadIdx.x >> 6;
-    const int wpb = blockDim.x >> 6;
+    const int wpb = P.wpb;
     // RX: one product slot per wave of the launch
     const int64_t eslot = blk * wpb + wave;
     if constexpr (G > 1) {
@@ -762,18 +762,14 @@ int launch_plane3_g(const StageParams &P, void *stream, int wpb)
         blocks = (waves + wpb - 1) / wpb;
         lds = (size_t)wpb * T::EPW * T::SLAB * sizeof(R);
     }
-    const dim3 grid((unsigned)blocks), block(64 * wpb);
-    hipStream_t st = static_cast<hipStream_t>(stream);
     if constexpr (stage_streams(3, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
-            hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX, G>), grid, block,
-                               lds, st, P);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
+            return launch_stage(&dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX, G>, blocks, wpb,
+                                lds, stream, P);
         }
     }
-    hipLaunchKernelGGL((dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX, G>), grid, block, lds, st,
-                       P);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_stage(&dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 0, RX, G>, blocks, wpb, lds,
+                        stream, P);
 }
 
 template <int NQ, int LAW, typename R, int GEO, int FLUX, int RX>

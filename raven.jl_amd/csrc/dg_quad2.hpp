@@ -313,8 +313,9 @@ __global__ void __launch_bounds__(256) dg_quad2_kernel(const StageParams P)
     extern __shared__ __attribute__((aligned(16))) unsigned char dg_lds[];
     const int grp = (int)(threadIdx.x / Q::LANES);
     const int gl = (int)(threadIdx.x - grp * Q::LANES);
-    const int gpb = (int)(blockDim.x / Q::LANES);
-    const int64_t blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int gpb = G > 1 ? 1 : P.wpb;
+    read_args<GEO, LAW, R>(P);
+    const int64_t blk = xcd_remap(blockIdx.x, P.blocks);
     R *glds = reinterpret_cast<R *>(dg_lds) + grp * Q::SLAB;
     quad2_clear_spare(glds, gl);
     quad2_group<NQ, LAW, R, FLUX, ST, G, V, GEO>(P, (blk * gpb + grp) * Q::CELLS, glds, gl);
@@ -333,17 +334,14 @@ int launch_quad2_v(const StageParams &P, void *stream, int wpb)
     const int64_t groups = (P.K + Q::CELLS - 1) / Q::CELLS;
     const int64_t blocks = (groups + gpb - 1) / gpb;
     const size_t lds = (size_t)gpb * Q::SLAB * sizeof(R);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid((unsigned)blocks), block(64 * wpb);
     if constexpr (stage_streams(2, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
-            hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>), grid, block, lds,
-                               st, P);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
+            return launch_stage(&dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>, blocks, wpb,
+                                lds, stream, P);
         }
     }
-    hipLaunchKernelGGL((dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>), grid, block, lds, st, P);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_stage(&dg_quad2_kernel<NQ, LAW, R, FLUX, 0, G, V, GEO>, blocks, wpb, lds,
+                        stream, P);
 }
 
 template <int NQ, int LAW, typename R, int FLUX, int GEO>

@@ -350,7 +350,7 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
     constexpr bool GEN = T::GEN, ADV = TP::ADV;
     __shared__ __align__(16) R lds[T::POOL];
     const int t = threadIdx.x;
-    const int64_t cell0 = xcd_remap(blockIdx.x, gridDim.x) * T::C;
+    const int64_t cell0 = xcd_remap(blockIdx.x, P.blocks) * T::C;
     const Law<DIM, LAW, R> law(P);
     const R *qin = static_cast<const R *>(P.q_in);
     // cells past the last one repeat its work and store nothing
@@ -805,7 +805,7 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
     __shared__ R lds[NV][T::NODE_THREADS];
     const int t = threadIdx.x;
     const int c = t / NP, node = t - c * NP;
-    const int64_t e = xcd_remap(blockIdx.x, gridDim.x) * T::NODE_C + c;
+    const int64_t e = xcd_remap(blockIdx.x, P.blocks) * T::NODE_C + c;
     const bool active = c < T::NODE_C && e < P.K;
     const Law<DIM, LAW, R> law(P);
     const R *qin = static_cast<const R *>(P.q_in);
@@ -1036,20 +1036,17 @@ __global__ void __launch_bounds__((FD<DIM, NQ, LAW, R, GEO, VF, SF>::NODE_THREAD
 }
 
 template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX, int ST>
-void launch_fd_st(const StageParams &P, hipStream_t st)
+int launch_fd_st(const StageParams &P, void *stream)
 {
     using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
     if constexpr (fd_has_line_kernel(DIM, LAW, VF)) {
         if (fd_by_line(DIM, NQ, LAW, (int)sizeof(R), VF, P.K)) {
-            hipLaunchKernelGGL((dg_fd_line_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>),
-                               dim3((unsigned)((P.K + T::C - 1) / T::C)), dim3(T::THREADS), 0, st,
-                               P);
-            return;
+            return launch_stage(&dg_fd_line_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>,
+                                (P.K + T::C - 1) / T::C, T::THREADS / 64, 0, stream, P);
         }
     }
-    hipLaunchKernelGGL((dg_fd_node_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>),
-                       dim3((unsigned)((P.K + T::NODE_C - 1) / T::NODE_C)), dim3(T::NODE_THREADS),
-                       0, st, P);
+    return launch_stage(&dg_fd_node_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>,
+                        (P.K + T::NODE_C - 1) / T::NODE_C, T::NODE_THREADS / 64, 0, stream, P);
 }
 
 template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX>
@@ -1057,15 +1054,11 @@ int launch_fd(const StageParams &P, void *stream, int)
 {
     if (P.K <= 0)
         return 0;
-    hipStream_t st = static_cast<hipStream_t>(stream);
     if constexpr (stage_streams(DIM, NQ, LAW, sizeof(R), GEO, VF)) {
-        if (P.streaming) {
-            launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, st);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
-        }
+        if (P.streaming)
+            return launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, stream);
     }
-    launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 0>(P, st);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 0>(P, stream);
 }
 
 template <int NQ, int LAW, int VF, int SF, bool RX>
