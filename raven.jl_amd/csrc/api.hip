@@ -104,6 +104,7 @@ struct rv_handle {
     MortarLauncher mortar = nullptr;
     int64_t mortar_cells = 0;
     int64_t *m_cells = nullptr, *m_partner = nullptr;
+    int64_t mortar_covered = 0;      // of them covered, listed first
     int64_t mortar_pairs = 0;        // non-conforming (cell, face) pairs,
     MortarPair *m_pairs = nullptr;  // covered sides first
     int32_t *m_kind = nullptr, *m_slot = nullptr;
@@ -1070,6 +1071,7 @@ int launch(rv_handle *h, const StageParams &P0, StageLauncher fn = nullptr)
         M.ncells = h->mortar_cells;
         M.cells = as_global(h->m_cells);
         M.npairs = h->mortar_pairs;
+        M.ncovered = h->mortar_covered;
         M.pairs = as_global(h->m_pairs);
         M.kind = as_global(h->m_kind);
         M.partner = as_global(h->m_partner);
@@ -1599,6 +1601,7 @@ int rv_enable_mortars(rv_handle *h, const int32_t *face_kind, const int64_t *par
             (k == 2 ? pairs : hanging).push_back(pr);
         }
     }
+    const int64_t ncovered = (int64_t)pairs.size();
     pairs.insert(pairs.end(), hanging.begin(), hanging.end());
     if (pairs.size() > (size_t)UINT32_MAX)
         return fail(h, RV_E_UNSUPPORTED, "too many non-conforming faces for one launch");
@@ -1632,6 +1635,7 @@ int rv_enable_mortars(rv_handle *h, const int32_t *face_kind, const int64_t *par
     HIP_TRY(h, hipStreamSynchronize(h->stream));
     h->mortar_cells = ncells;
     h->mortar_pairs = npairs;
+    h->mortar_covered = ncovered;
     h->mortar = ml;
     return RV_OK;
 }

@@ -196,7 +196,7 @@ struct MortarParams {
     const int64_t RV_GLOBAL *cells;
     // their non-conforming (cell, face) pairs: covered (coarse) sides first,
     // which take longer, then hanging (fine) sides
-    int64_t npairs;
+    int64_t npairs, ncovered;
     const MortarPair RV_GLOBAL *pairs;
     const int32_t RV_GLOBAL *kind;     // (K, 2dim): 0 conforming, 1 hanging, 2 covered
     const int64_t RV_GLOBAL *partner;  // (K, 2dim, 4), see forest_mortars
