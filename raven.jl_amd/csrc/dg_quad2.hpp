@@ -17,7 +17,7 @@
 //    share one workgroup's cells (5, 7, 5 cells over 128, 256, 256 lanes) and
 //    synchronise with workgroup barriers (so do batches launching a kind on
 //    its own); the batches' work-list kernel uses G = 1;
-//  * light cells (advection, FP32 Euler) of a grid that fills the device give
+//  * light cells (advection of grids that fill the device, FP32 Euler) give
 //    a lane V = 4 or 2 nodes, one in each of V sets of cells, all requested
 //    before the first wait: a wave then has V times the bytes in flight;
 //  * curved cells publish contravariant fluxes and lifted numerical fluxes.
@@ -360,9 +360,11 @@ int launch_quad2(const StageParams &P, void *stream, int wpb)
     // waves per CU (256 CUs).  FP64 advection, us per LSRK stage, V nodes / one:
     // Nq = 5 on 16^2 4.98 / 2.95, 96^2 (3687 waves) 5.81 / 4.78, 128^2 (6554)
     // 6.86 / 6.32, 192^2 (14746) 9.94 / 11.0; Nq = 8 on 64^2 (4096) 5.64 / 5.10,
-    // 96^2 (9216) 7.77 / 8.81.  FP32 Euler, Nq = 5: 5.40 / 3.99 on 16^2, even
-    // from 96^2 on.
-    if constexpr (V > 1) {
+    // 96^2 (9216) 7.77 / 8.81.  Not FP32 Euler (5.40 / 3.99 on 16^2): there the
+    // compiler fuses the multiplications and additions of one and of two nodes
+    // differently, and a batch's members, which have two, give the bits of the
+    // operator alone.
+    if constexpr (LAW == LAW_ADVECTION && V > 1) {
         constexpr int cells = 64 * G / (NQ * NQ);
         if (!P.streaming && (P.K + cells - 1) / cells * G <= 6144)
             return launch_quad2_v<NQ, LAW, R, FLUX, GEO, 1>(P, stream, wpb);

@@ -93,3 +93,34 @@ def test_2d_nodes_per_lane(torch, R, nq, law, dtype):
     line = 64 * waves // nq**2 * (6144 // waves)
     for K in (line, line + 1, line + 37):
         check_stage(torch, R, 2, nq, [K, 1], law, dtype, "auto")
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("nq", range(2, 9))
+def test_2d_small_advection_in_a_batch(torch, R, nq, dtype):
+    """One node per lane (the operator alone on a small grid) and four (the
+    batch's kernels, a work list and a launch of the kind's own) give the same
+    bits: random states, a and b_dt away from zero."""
+    rng = np.random.default_rng(nq)
+    dgs, states = [], []
+    for n in ([3, 2], [40, 41]):
+        gm = R.GridManager(R.LobattoCell(nq, nq),
+                           R.brick([PB.julia_range(-1, 1, k + 1) for k in n], (True, False)))
+        dg = R.DGSEM(law=R.AdvectionLaw(2, [1.0, 0.7]), grid=R.generate(gm), dtype=dtype)
+        dgs.append(dg)
+        states.append([torch.from_numpy(rng.standard_normal((dg.K, dg.ns, dg.Np)))
+                       .to(dg.torch_dtype).cuda() for _ in range(2)])
+    want = []
+    for dg, (q, d) in zip(dgs, states):
+        qo, dq = torch.empty_like(q), d.clone()
+        dg.lsrk_stage(qo, q, dq, -0.7, 3e-3)
+        want.append((qo, dq))
+    batch = R.Batch(dgs)
+    for items in (1, 1 << 30):  # every kind on its own; all in the work list
+        batch.configure(own_launch_items=items)
+        qo, dq = [torch.empty_like(q) for q, _ in states], [d.clone() for _, d in states]
+        batch.stage(qo, [q for q, _ in states], dq, [-0.7] * 2, [3e-3] * 2)
+        torch.cuda.synchronize()
+        for k in range(2):
+            assert torch.equal(qo[k], want[k][0]) and torch.equal(dq[k], want[k][1])
+    batch.close()
