@@ -449,10 +449,11 @@ __global__ void __launch_bounds__(256) dg_stage_kernel_1d(const StageParams P)
     stage_wave_1d<NQ, LAW, R, GEO, FLUX, ST>(P, (blk * P.wpb + wave) * (64 / NQ), lds[wave]);
 }
 
-// Launch a stage kernel of wpb waves per workgroup; 0, or -1 with HIP's error left for the caller.  A
-// small stage takes less than its launch, so the launch is one runtime call: the
-// <<<>>> syntax makes two (it puts the shape aside and fetches it back) and
-// then asks for the last error, 2.71 against 2.55 us on the host.
+// Launch a stage kernel of wpb waves per workgroup; 0, or -1 with HIP's error
+// left for the caller.  A small stage takes less than its launch, so the launch
+// is one runtime call: the <<<>>> syntax makes two (it puts the shape aside and
+// fetches it back) and then the last error was asked for, 2.71 against 2.55 us
+// on the host.
 inline int launch_stage(void (*kernel)(StageParams), int64_t blocks, int wpb, size_t lds,
                         void *stream, const StageParams &P0)
 {
