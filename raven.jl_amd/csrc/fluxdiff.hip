@@ -74,6 +74,7 @@ template <typename R>
 struct LogSeries {
     static constexpr int TERMS[2] = {sizeof(R) == 8 ? 8 : 4, sizeof(R) == 8 ? 4 : 2};
     static constexpr double LIMIT[2] = {1e-2, 1e-4};
+    static constexpr double FLIMIT[2] = {1e-1, 1e-2};  // the same for f
     double f[8], g[8];
     constexpr LogSeries() : f{}, g{}
     {
@@ -527,13 +528,16 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
         // Which log series serves every pair of the wave's lines: a pair's f is
         // at most that of the line's extremes.  The extremes are taken on the
         // leading 32 bits (positive values order as their bits do; a negative
-        // or NaN value fails the test), the largest rounded up.
+        // or NaN value fails the test), the largest rounded up.  They are
+        // compared without squares, which would leave the type's range, and
+        // each is kept where the flux's reciprocals are normal numbers (FP64
+        // takes one of the product of the sums of rho and of b).
         int rough = 0;  // 0: short series, 1: long series, 2: logarithms
         if constexpr (TP::EC) {
             constexpr int W = sizeof(R) / 4;  // 32-bit words per value
+            constexpr R LEAST = W == 2 ? R(1e-140) : R(1e-37), MOST = W == 2 ? R(1e140) : R(1e37);
             const uint32_t *w = reinterpret_cast<const uint32_t *>(lds) + W * lbase + (W - 1);
             bool ok[2] = {true, true};
-            R least = R(1), most = R(1);  // of rho times b (see TwoPoint::flux)
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 uint32_t lo = w[W * k * CMP], hi = lo;
@@ -551,14 +555,12 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
                     x0 = __uint_as_float(lo);
                     x1 = __uint_as_float(hi);
                 }
-                least = least * x0, most = most * x1;
-                const R d = (x1 - x0) * (x1 - x0), s = (x1 + x0) * (x1 + x0);
+                const R d = fabs(x1 - x0), s = x1 + x0;
+                ok[0] = ok[0] && x0 > LEAST && x1 < MOST;
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    ok[j] = ok[j] && d < R(LogSeries<R>::LIMIT[j]) * s;
+                    ok[j] = ok[j] && d < R(LogSeries<R>::FLIMIT[j]) * s;
             }
-            if constexpr (W == 2)
-                ok[0] = ok[0] && least > R(1e-290) && most < R(1e290);
             ok[1] = ok[1] && ok[0];
             rough = __all(ok[1]) ? 0 : __all(ok[0]) ? 1 : 2;
         }
