@@ -39,7 +39,11 @@
 //
 // The node kernel (fd_stage_node; everything else): a lane per node, each pair
 // evaluated from both ends.  The fluxes of the central forms cost little, and
-// small grids wait for the chain of one wave.
+// small grids wait for the chain of one wave.  Pairs that need logarithms cost
+// most: with log_factor in place of the library's logarithm, 375000 1-D cells of
+// Nq = 8 with such states take 157 us a FP64 stage (216 us without it), 56^2 of
+// Nq = 8 32 (43); its registers make stages of smooth states on grids near the
+// switch up to 10 % longer (7^3 of Nq = 8 25.9 -> 28.5).
 //
 // A relaxation stage (RX, the RLSRK step of odesolvers.jl:117-151) keeps
 // k = L(q) apart from a dq, forms dq = a dq + k at the end and leaves each
@@ -132,34 +136,14 @@ __device__ __forceinline__ float recip(float x)
     return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
 
-// ... and with a division's values for zero, infinity and NaN (one instruction
-// more; the division itself made small grids' stages 15 % longer)
-__device__ __forceinline__ double recip_any(double x)
+// r = recip(x) with a division's values for zero, infinity and NaN
+__device__ __forceinline__ double recip_any(double x, double r)
 {
-    return __builtin_amdgcn_div_fixup(recip(x), x, 1.0);
+    return __builtin_amdgcn_div_fixup(r, x, 1.0);
 }
-__device__ __forceinline__ float recip_any(float x)
+__device__ __forceinline__ float recip_any(float x, float r)
 {
-    return __builtin_amdgcn_div_fixupf(recip(x), x, 1.0f);
-}
-
-__device__ __forceinline__ bool positive_normal(double x)
-{
-    return __builtin_amdgcn_class(x, 0x100);
-}
-__device__ __forceinline__ bool positive_normal(float x)
-{
-    return __builtin_amdgcn_classf(x, 0x100);
-}
-__device__ __forceinline__ double mantissa(double x, int &e)
-{
-    e = __builtin_amdgcn_frexp_exp(x);
-    return __builtin_amdgcn_frexp_mant(x);
-}
-__device__ __forceinline__ float mantissa(float x, int &e)
-{
-    e = __builtin_amdgcn_frexp_expf(x);
-    return __builtin_amdgcn_frexp_mantf(x);
+    return __builtin_amdgcn_div_fixupf(r, x, 1.0f);
 }
 
 // F = log(a / b) / 2f beyond the series, or (INV) 1 / 2F; s = a + b, d = a - b,
@@ -307,33 +291,33 @@ struct TwoPoint {
                 const R i = recip(sr * sb);
                 isr = i * sb;
                 isb = i * sr;
-            } else if constexpr (SERIES >= 0) {
+            } else {
                 isr = recip(sr);
                 isb = recip(sb);
-            } else {
-                isr = recip_any(sr);
-                isb = recip_any(sb);
             }
             const R fr = dr * isr, fb = db * isb;
             const R ur = fr * fr, ub = fb * fb;
             R G, Fb;  // 1 / 2F of rho, F of b
-            if constexpr (SERIES < 0) {
-                // the logarithm beyond the series
-                if (ur < R(LogSeries<R>::LIMIT[0]))
-                    G = series_g<R, 0>(ur);
-                else if constexpr (SERIES == -2)
-                    G = log_factor<true>(a.rho, b.rho, sr, dr, isr);
-                else
-                    G = fr / log(a.rho / b.rho);
-                if (ub < R(LogSeries<R>::LIMIT[0]))
-                    Fb = series_f<R, 0>(ub);
-                else if constexpr (SERIES == -2)
-                    Fb = log_factor<false>(a.b, b.b, sb, db, isb);
-                else
-                    Fb = log(a.b / b.b) / (R(2) * fb);
-            } else {
+            if constexpr (SERIES >= 0) {
                 G = series_g<R, SERIES>(ur);
                 Fb = series_f<R, SERIES>(ub);
+            } else {
+                // the logarithm beyond the series; there a sum that is zero or
+                // infinite (its f is NaN) divides as a division would
+                if (ur < R(LogSeries<R>::LIMIT[0])) {
+                    G = series_g<R, 0>(ur);
+                } else {
+                    isr = recip_any(sr, isr);
+                    G = SERIES == -2 ? log_factor<true>(a.rho, b.rho, sr, dr, isr)
+                                     : dr * isr / log(a.rho / b.rho);
+                }
+                if (ub < R(LogSeries<R>::LIMIT[0])) {
+                    Fb = series_f<R, 0>(ub);
+                } else {
+                    isb = recip_any(sb, isb);
+                    Fb = SERIES == -2 ? log_factor<false>(a.b, b.b, sb, db, isb)
+                                      : log(a.b / b.b) / (R(2) * (db * isb));
+                }
             }
             R ua[DIM];
 #pragma unroll
@@ -695,13 +679,18 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
             pairs(std::integral_constant<int, 0>{});
         } else if constexpr (TP::EC) {
             // a rolled loop (its indexes are the same on every lane): the
-            // accumulators are addressed by weights that are zero elsewhere
+            // accumulators are addressed by weights that are zero elsewhere,
+            // by the partner's only where registers allow the outer loop to
+            // be unrolled (2-D, Nq = 7, 12321 curved cells, FP64: 75.7 ->
+            // 74.1 us a stage; 3-D cells then spill: Nq = 8, 18^3, 136 ->
+            // 155 us without a logarithm)
+            constexpr int UNROLL = DIM == 2 && NQ >= 6 ? NQ : 1;
 #pragma unroll
             for (int n = 0; n < NQ; ++n)
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
                     acc[n][s] = R(0);
-#pragma unroll 1
+#pragma unroll(UNROLL)
             for (int i = 0; i + 1 < NQ; ++i) {
                 const Node a = load(i);
                 R la[DIM];
@@ -726,6 +715,8 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
                     }
 #pragma unroll
                     for (int k = 0; k < NQ; ++k) {
+                        if (UNROLL > 1 && k < i)
+                            continue;
                         const R w = k == i ? wi : k == n ? wn : R(0);
 #pragma unroll
                         for (int s = 0; s < NS; ++s)
