@@ -877,7 +877,11 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
     using TP = typename T::TP;
     constexpr int NS = T::NS, NP = T::NP, NL = T::NL, NF = T::NF, NV = TP::NV;
     constexpr bool GEN = T::GEN;
-    __shared__ R lds[NV][T::NODE_THREADS];
+    // advection on curved cells: a node's u . l_d, so that a pair reads its
+    // partner's from LDS and not the partner's metric terms from memory (curved
+    // 24^3 cells of Nq = 6, FP64: 213 -> 141 us a stage)
+    constexpr bool UL = GEN && TP::ADV;
+    __shared__ R lds[NV + (UL ? DIM : 0)][T::NODE_THREADS];
     const int t = threadIdx.x;
     const int c = t / NP, node = t - c * NP;
     const int64_t e = xcd_remap(blockIdx.x, P.blocks) * T::NODE_C + c;
@@ -898,7 +902,7 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
 
     // the node's own loads, and the neighbour states of the faces it lies on
     // (one per direction: Nq > 1)
-    R q[NS], x[NV], qp[DIM][NS], dqo[NS], mji = R(1);
+    R q[NS], x[NV], qp[DIM][NS], dqo[NS], mji = R(1), ul[DIM];
     double mj = 0.0;
     bool on_face[DIM];
     int side[DIM], m[DIM];
@@ -932,6 +936,17 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
 #pragma unroll
         for (int k = 0; k < NV; ++k)
             lds[k][t] = x[k];
+        if constexpr (UL) {
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                const int64_t g = ((e * DIM + d) * DIM) * NP + node;
+                ul[d] = law.u[0] * R(vgeo[g]);
+#pragma unroll
+                for (int j = 1; j < DIM; ++j)
+                    ul[d] = ul[d] + law.u[j] * R(vgeo[g + j * NP]);
+                lds[NV + d][t] = ul[d];
+            }
+        }
 #pragma unroll
         for (int d = 0; d < DIM; ++d)
             if (on_face[d]) {
@@ -981,7 +996,7 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
             const int stride = d == 0 ? 1 : d == 1 ? NQ : NQ * NQ;
             const int64_t g = ((e * DIM + d) * DIM) * NP + node;
             R la[DIM], kd[NS];
-            if constexpr (GEN) {
+            if constexpr (GEN && !UL) {
 #pragma unroll
                 for (int j = 0; j < DIM; ++j)
                     la[j] = R(vgeo[g + j * NP]);
@@ -1001,13 +1016,18 @@ __device__ __forceinline__ void fd_stage_node(const StageParams &P)
                 if constexpr (GEN) {
                     const R *D = tab + NQ * NQ;
                     const R Dni = D[n * NQ + i], Din = D[i * NQ + n];
+                    if constexpr (UL) {
+                        F[0] = R(0.5) * (Dni * lds[NV + d][t + to] - Din * ul[d]) * (ad.rho + y[0]);
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < DIM; ++j)
-                        mv[j] = Dni * R(vgeo[g + to + j * NP]) - Din * la[j];
+                        for (int j = 0; j < DIM; ++j)
+                            mv[j] = Dni * R(vgeo[g + to + j * NP]) - Din * la[j];
+                    }
                 } else {
                     w = tab[i * NQ + n];
                 }
-                TP::template flux<-2>(lawd, ad, turned(TP::node(law, y)), mv, F);
+                if constexpr (!UL)
+                    TP::template flux<-2>(lawd, ad, turned(TP::node(law, y)), mv, F);
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
                     kd[s] = kd[s] + w * F[s];
