@@ -230,9 +230,15 @@ constexpr int fd_node_cells(int dim, int nq)
     const int most = dim == 1 ? 64 : 256;
     return np >= most ? 1 : most / np;
 }
-constexpr bool fd_has_line_kernel(int dim, int law, int vflux)
+// The line kernel's forms.  Not 2-D Nq = 2 in FP32: two lines of one pair each
+// are less work than the sums that move between directions, and twice as many
+// lanes hide the faces' reads (us per stage, line / node: 387^2 cells Rusanov
+// 26.2 / 16.1, own flux 18.5 / 16.3, curved 33.0 / 18.0 and 24.8 / 17.4; 1414^2 291
+// / 192; in FP64 224^2 own flux 8.4 / 9.3, 612^2 Rusanov 52.5 / 47.3).
+constexpr bool fd_has_line_kernel(int dim, int nq, int law, int real_bytes, int vflux)
 {
-    return dim > 1 && law == LAW_EULER && vflux == FLUX_EC;
+    return dim > 1 && law == LAW_EULER && vflux == FLUX_EC &&
+           !(dim == 2 && nq == 2 && real_bytes == 4);
 }
 // Whether a launch over K cells takes the line kernel: from about one wave per
 // SIMD of the device on (FP64; FP32, whose chains are shorter, from 1.75).
@@ -245,7 +251,7 @@ constexpr bool fd_has_line_kernel(int dim, int law, int vflux)
 // 20.7; 24^3 FP64 315 / 658, FP32 185 / 260.
 inline bool fd_by_line(int dim, int nq, int law, int real_bytes, int vflux, int64_t K)
 {
-    if (!fd_has_line_kernel(dim, law, vflux))
+    if (!fd_has_line_kernel(dim, nq, law, real_bytes, vflux))
         return false;
     const int c = fd_cells_per_workgroup(dim, nq);
     const int waves = (c * dim * (dim == 2 ? nq : nq * nq) + 63) / 64;

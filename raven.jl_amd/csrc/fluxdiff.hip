@@ -1134,7 +1134,7 @@ template <int DIM, int NQ, int LAW, typename R, int GEO, int VF, int SF, bool RX
 int launch_fd_st(const StageParams &P, void *stream)
 {
     using T = FD<DIM, NQ, LAW, R, GEO, VF, SF>;
-    if constexpr (fd_has_line_kernel(DIM, LAW, VF)) {
+    if constexpr (fd_has_line_kernel(DIM, NQ, LAW, (int)sizeof(R), VF)) {
         if (fd_by_line(DIM, NQ, LAW, (int)sizeof(R), VF, P.K)) {
             return launch_stage(&dg_fd_line_kernel<DIM, NQ, LAW, R, GEO, VF, SF, RX, ST>,
                                 (P.K + T::C - 1) / T::C, T::THREADS / 64, 0, stream, P);
