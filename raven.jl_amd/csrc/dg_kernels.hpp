@@ -449,6 +449,69 @@ __global__ void __launch_bounds__(256) dg_stage_kernel_1d(const StageParams P)
     stage_wave_1d<NQ, LAW, R, GEO, FLUX, ST>(P, (blk * P.wpb + wave) * (64 / NQ), lds[wave]);
 }
 
+// The right-hand side alone of FP32 advection on large 1-D grids: a lane per
+// cell.  A node is four bytes, and with no q_out written what a wave does besides
+// counts most: here the operator is uniform (scalar loads) and a cell's fluxes
+// stay in its lane.  us per right-hand side, a lane per node / per cell: 600000
+// cells of Nq = 5 15.0 / 9.3, 375000 of Nq = 8 17.9 / 12.0, 62500 4.5 / 4.2, below
+// the same; FP64, whose strided lanes fetch twice the lines, 375000 of Nq = 8 20.1
+// / 21.8, 500000 of Nq = 6 15.3 / 19.0.
+constexpr int64_t CELL_NODES_1D = 400000;
+template <int NQ, int LAW, typename R, int GEO, int FLUX>
+__global__ void __launch_bounds__(64) dg_rhs_cell_kernel_1d(const StageParams P)
+{
+    using S = Stage<1, NQ, LAW, R, GEO, FLUX>;
+    static_assert(S::NS == 1, "advection");
+    constexpr bool GEN = GEO == GEO_GENERAL;
+    const int64_t e = xcd_remap(blockIdx.x, P.blocks) * 64 + threadIdx.x;
+    if (e >= P.K)
+        return;
+    const Law<1, LAW, R> law(P);
+    const R *qin = static_cast<const R *>(P.q_in);
+    R *dq = static_cast<R *>(P.dq) + e * NQ;
+    R q[NQ], f[NQ], qp[2], nf[2];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+        q[n] = qin[e * NQ + n];
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+        S::neighbour_state(P, qin, e, side, 0, q + (side ? NQ - 1 : 0), qp + side);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+        law.flux_row(0, q + n, f + n);
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        const int end = side ? NQ - 1 : 0;
+        if constexpr (GEN) {
+            const R nv[1] = {R(P.sgeo[(e * 2 + side) * 2])};
+            S::nflux_general(law, nv, q + end, qp + side, nf + side);
+            nf[side] = R(P.sgeo[(e * 2 + side) * 2 + 1]) * nf[side];
+        } else {
+            S::nflux_axis(law, 0, side ? R(1) : R(-1), f + end, q + end, qp + side, nf + side);
+            nf[side] = R(P.winv[end]) * nf[side];
+        }
+    }
+    if constexpr (GEN) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+            f[n] = R(P.vgeo[e * NQ + n]) * f[n];
+    }
+    const double RV_GLOBAL *M = GEN ? P.Dt : P.Dw;
+    const bool on = P.dir_mask & 1;
+    const R a = R(P.a);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        R x = R(M[i * NQ]) * f[0];
+#pragma unroll
+        for (int n = 1; n < NQ; ++n)
+            x = x + R(M[i * NQ + n]) * f[n];
+        if (i == 0 || i == NQ - 1)
+            x = x - nf[i != 0];
+        x = on ? R(GEN ? P.mji[e * NQ + i] : P.affine[e]) * x : R(0);
+        dq[i] = P.read_dq ? a * dq[i] + x : x;
+    }
+}
+
 // Launch a stage kernel of wpb waves per workgroup; 0, or -1 with HIP's error
 // left for the caller.  A small stage takes less than its launch, so the launch
 // is one runtime call: the <<<>>> syntax makes two (it puts the shape aside and
@@ -474,6 +537,12 @@ int launch_stage_1d(const StageParams &P, void *stream, int wpb)
         return 0;
     if (wpb != 1 && wpb != 2 && wpb != 4)
         wpb = 1;
+    if constexpr (LAW == LAW_ADVECTION && sizeof(R) == 4) {
+        if (!P.write_q && P.K * NQ > CELL_NODES_1D) {
+            return launch_stage(&dg_rhs_cell_kernel_1d<NQ, LAW, R, GEO, FLUX>, (P.K + 63) / 64, 1,
+                                0, stream, P);
+        }
+    }
     const int64_t cells = (int64_t)wpb * (64 / NQ);
     const int64_t blocks = (P.K + cells - 1) / cells;
     if constexpr (stage_streams(1, NQ, LAW, sizeof(R), GEO, 0)) {
