@@ -123,7 +123,7 @@ typedef struct rv_info {
     int32_t geometry;           /* resolved RV_GEOM_AFFINE or RV_GEOM_GENERAL */
     int32_t faces_self;         /* faces with q+ = q- (boundary or self-mapped) */
     int32_t faces_explicit;     /* faces needing per-node neighbour indices */
-    int32_t streaming;          /* 1: stages stream dq and q_out past L2 (3 states > 256 MB, written in whole lines) */
+    int32_t streaming;          /* 1: stages stream dq and q_out past L2 (3 states > 256 MB, where that measured faster) */
     int64_t ncells;
     int64_t state_bytes;        /* bytes of one state array */
     int64_t device_bytes;       /* device memory held by the handle */

@@ -1023,7 +1023,16 @@ int create_from_desc(const rv_desc *d, rv_handle *h)
     return finish_setup(h, d->D, d->weights);
 }
 
-constexpr int64_t STREAM_BYTES = (int64_t)256 << 20;
+// whether a stage (write_q), or a right-hand side alone, streams dq and q_out
+// past L2 (which then keeps the q lines that face reads share)
+int16_t streams(const rv_handle *h, bool write_q)
+{
+    const int b = h->dtype == RV_F32 ? 4 : 8;
+    return launch_streams(h->dim, h->nq, h->law, b, h->geo, h->vflux, write_q,
+                          h->Np * h->ns * h->K * b)
+               ? 1
+               : 0;
+}
 
 StageParams stage_params(rv_handle *h)
 {
@@ -1048,20 +1057,14 @@ StageParams stage_params(rv_handle *h)
     P.gamma = h->gamma;
     for (int c = 0; c < 3; ++c)
         P.u[c] = h->u[c];
-    // a stage touches q_in, dq and q_out; beyond the 256 MB Infinity Cache of
-    // MI355X nothing of dq and q_out survives to the next stage, so kernels
-    // that write whole lines (stage_streams) stream them past L2 (which then
-    // keeps the q lines that face reads share)
-    const int b = h->dtype == RV_F32 ? 4 : 8;
-    const int64_t state = h->Np * h->ns * h->K * b;
-    P.streaming =
-        3 * state > STREAM_BYTES && stage_streams(h->dim, h->nq, h->law, b, h->geo, h->vflux) ? 1 : 0;
+    P.streaming = streams(h, true);
     return P;
 }
 
 int launch(rv_handle *h, const StageParams &P0, StageLauncher fn = nullptr)
 {
     StageParams P = P0;
+    P.streaming = streams(h, P.write_q);
     MortarParams M{};
     // the 3-D weak-form column kernel adds the mortar updates after its own
     // stores; the other stage kernels leave that to mortar_apply_kernel

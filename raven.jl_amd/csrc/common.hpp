@@ -108,9 +108,10 @@ struct StageParams {
 // 448, FP32 412 / 272, Nq = 7 FP32 32^3 316 / 256; 2-D Nq = 8 FP64 390^2 274 /
 // 286, Nq = 4 FP32 760^2 198 / 167, Nq = 5 FP64 620^2 356 / 318; entropy-
 // conservative form, 2-D Nq = 5 FP64 620^2 385 / 351, curved 3-D Nq = 5 FP32
-// 40^3 380 / 367.  On 3-D affine cells whole 32-byte sectors (Nq = 6 FP64 30^3
-// 227 / 241, 38^3 474 / 462; curved 394 / 377, 794 / 729), and for flux
-// differencing any cell (Nq = 5 FP64 40^3 376 / 402), are enough.
+// 40^3 380 / 367.  On 3-D affine cells whole 32-byte sectors are enough up to
+// about 30^3 cells of Nq = 6 and cost little beyond (FP64 30^3 227 / 241, 38^3 474 /
+// 462; not curved ones: 394 / 377, 794 / 729), and for flux differencing any cell
+// (Nq = 5 FP64 40^3 376 / 402).
 constexpr bool stage_streams(int dim, int nq, int law, int real_bytes, int geo, int vflux)
 {
     if (law == LAW_ADVECTION)
@@ -118,6 +119,52 @@ constexpr bool stage_streams(int dim, int nq, int law, int real_bytes, int geo, 
     const bool brick3 = dim == 3 && geo == GEO_AFFINE;
     const int piece = (dim == 1 ? nq : dim == 3 && vflux ? nq * nq * nq : nq * nq) * real_bytes;
     return piece % (brick3 && vflux ? 1 : brick3 ? 32 : 128) == 0;
+}
+
+// The Infinity Cache.  A stage touches three states; beyond this in all nothing
+// of dq and q_out survives to the next one.
+constexpr int64_t CACHE_BYTES = (int64_t)256 << 20;
+
+// ... and weak-form brick launches that stream although their pieces end inside
+// lines.  While one state fits the cache, streaming the others leaves q there:
+// that is worth the partial writes where pieces are long, and to a right-hand
+// side alone, which writes only dq.  us, streamed / not, state in MB: right-hand
+// sides 2-D Nq = 6 FP64 122 73.1 / 75.4, 244 135 / 170, Nq = 7 FP64 244 148 / 183,
+// Nq = 6 FP32 100 70.3 / 67.5, 122 86 / 96, Nq = 4 FP32 122 83 / 97, 200 134 / 166,
+// but 244 215 / 202, Nq = 5 FP64 244 172 / 184, 488 368 / 361, Nq = 3 FP64 100 77.5 /
+// 71.3, 155 118 / 135, 244 236 / 212; 3-D Nq = 5 FP64 156 110 / 121, 305 228 / 230,
+// 596 458 / 435, Nq = 7 FP64 159 161 / 153; stages 2-D Nq = 6 FP64 122 126 / 132, 244
+// 247 / 255, 489 520 / 504, Nq = 5 FP64 244 298 / 281.
+constexpr bool resident_streams(int dim, int nq, int law, int geo, int real_bytes, int vflux,
+                                bool write_q, int64_t state)
+{
+    if (law == LAW_ADVECTION || geo != GEO_AFFINE || vflux || dim == 1)
+        return false;
+    const int piece = nq * nq * real_bytes;
+    if (write_q)
+        return dim == 2 && piece >= 288 && state <= CACHE_BYTES;
+    // (below, q and dq fit the cache together)
+    if (20 * state <= 9 * CACHE_BYTES)
+        return false;
+    if (dim == 2)
+        return piece >= 64 && state <= (piece >= 128 ? CACHE_BYTES : CACHE_BYTES / 6 * 5);
+    return piece >= 128 && nq <= 6 && (state <= CACHE_BYTES || piece % 16 == 0);
+}
+
+// Whether a launch streams, and whether any launch of a form does (its streaming
+// variant is then built).
+inline bool launch_streams(int dim, int nq, int law, int real_bytes, int geo, int vflux,
+                           bool write_q, int64_t state)
+{
+    return 3 * state > CACHE_BYTES &&
+           (stage_streams(dim, nq, law, real_bytes, geo, vflux) ||
+            resident_streams(dim, nq, law, geo, real_bytes, vflux, write_q, state));
+}
+constexpr bool form_streams(int dim, int nq, int law, int real_bytes, int geo, int vflux)
+{
+    return stage_streams(dim, nq, law, real_bytes, geo, vflux) ||
+           resident_streams(dim, nq, law, geo, real_bytes, vflux, false, CACHE_BYTES / 2) ||
+           resident_streams(dim, nq, law, geo, real_bytes, vflux, true, 0);
 }
 
 // Waves of a workgroup of the 3-D column kernel that packs its cells across
@@ -136,19 +183,21 @@ constexpr int plane3_pack_waves(int nq) { return nq == 5 ? 2 : nq == 6 || nq == 
 // FP32 42.7 / 39.9, curved FP64 146 / 140, 32^3 FP64 549 / 520, curved 921 / 802, FP32
 // 256 / 235; Nq = 5 10^3 FP64 12.1 / 14.1, 44^3 FP64 448 / 445, FP32 272 / 260, curved
 // FP32 408 / 385, FP64 717 / 698.
-inline bool plane3_packed(int nq, int law, int real_bytes, int geo, int64_t K)
+inline bool plane3_packed(int nq, int law, int real_bytes, int geo, int64_t K, bool write_q)
 {
     if (plane3_pack_waves(nq) == 1)
         return false;
     const int ns = law == LAW_ADVECTION ? 1 : 5;
-    const bool large = 3 * K * nq * nq * nq * ns * real_bytes > ((int64_t)256 << 20);
+    const bool large = 3 * K * nq * nq * nq * ns * real_bytes > CACHE_BYTES;
     const bool curved = geo != GEO_AFFINE;
     if (nq == 5)
-        return !(large && (real_bytes == 4 || curved));
+        return !(large && ((real_bytes == 4 && write_q) || curved));
     if (K <= (nq == 6 ? 1024 : 2048))
         return false;
+    // (a right-hand side alone writes less and waits less: FP32 29^3 75.6 / 89.4
+    // us, 36^3 137 / 172, 49^3 399 / 445)
     if (nq == 6)
-        return !(large && real_bytes == 4);
+        return !(large && real_bytes == 4 && (write_q || curved));
     return real_bytes == 8 && !curved && !large;
 }
 
@@ -159,7 +208,7 @@ inline bool plane3_packed(int nq, int law, int real_bytes, int geo, int64_t K)
 inline int64_t plane3_relax_slots(int nq, int law, int real_bytes, int geo, int64_t K, int wpb)
 {
     const int nq2 = nq * nq;
-    if (plane3_packed(nq, law, real_bytes, geo, K)) {
+    if (plane3_packed(nq, law, real_bytes, geo, K, true)) {
         const int g = plane3_pack_waves(nq), cpg = 64 * g / nq2;
         return (K + cpg - 1) / cpg * g;
     }

@@ -545,7 +545,7 @@ int launch_stage_1d(const StageParams &P, void *stream, int wpb)
     }
     const int64_t cells = (int64_t)wpb * (64 / NQ);
     const int64_t blocks = (P.K + cells - 1) / cells;
-    if constexpr (stage_streams(1, NQ, LAW, sizeof(R), GEO, 0)) {
+    if constexpr (form_streams(1, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
             return launch_stage(&dg_stage_kernel_1d<NQ, LAW, R, GEO, FLUX, 1>, blocks, wpb, 0,
                                 stream, P);

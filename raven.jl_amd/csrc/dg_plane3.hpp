@@ -762,7 +762,7 @@ int launch_plane3_g(const StageParams &P, void *stream, int wpb)
         blocks = (waves + wpb - 1) / wpb;
         lds = (size_t)wpb * T::EPW * T::SLAB * sizeof(R);
     }
-    if constexpr (stage_streams(3, NQ, LAW, sizeof(R), GEO, 0)) {
+    if constexpr (form_streams(3, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
             return launch_stage(&dg_plane3_kernel<NQ, LAW, R, GEO, FLUX, 1, RX, G>, blocks, wpb,
                                 lds, stream, P);
@@ -779,7 +779,7 @@ int launch_plane3_rx(const StageParams &P, void *stream, int wpb)
     if (P.K <= 0)
         return 0;
     if constexpr (G > 1) {
-        if (plane3_packed(NQ, LAW, sizeof(R), GEO, P.K))
+        if (plane3_packed(NQ, LAW, sizeof(R), GEO, P.K, P.write_q))
             return launch_plane3_g<NQ, LAW, R, GEO, FLUX, RX, G>(P, stream, wpb);
     }
     return launch_plane3_g<NQ, LAW, R, GEO, FLUX, RX, 1>(P, stream, wpb);

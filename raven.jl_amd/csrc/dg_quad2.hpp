@@ -334,7 +334,7 @@ int launch_quad2_v(const StageParams &P, void *stream, int wpb)
     const int64_t groups = (P.K + Q::CELLS - 1) / Q::CELLS;
     const int64_t blocks = (groups + gpb - 1) / gpb;
     const size_t lds = (size_t)gpb * Q::SLAB * sizeof(R);
-    if constexpr (stage_streams(2, NQ, LAW, sizeof(R), GEO, 0)) {
+    if constexpr (form_streams(2, NQ, LAW, sizeof(R), GEO, 0)) {
         if (P.streaming) {
             return launch_stage(&dg_quad2_kernel<NQ, LAW, R, FLUX, 1, G, V, GEO>, blocks, wpb,
                                 lds, stream, P);

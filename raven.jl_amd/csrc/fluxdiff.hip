@@ -1149,7 +1149,7 @@ int launch_fd(const StageParams &P, void *stream, int)
 {
     if (P.K <= 0)
         return 0;
-    if constexpr (stage_streams(DIM, NQ, LAW, sizeof(R), GEO, VF)) {
+    if constexpr (form_streams(DIM, NQ, LAW, sizeof(R), GEO, VF)) {
         if (P.streaming)
             return launch_fd_st<DIM, NQ, LAW, R, GEO, VF, SF, RX, 1>(P, stream);
     }
