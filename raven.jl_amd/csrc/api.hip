@@ -1103,18 +1103,22 @@ int launch(rv_handle *h, const StageParams &P0, StageLauncher fn = nullptr)
 }
 
 // Sums over the states (reduce_kernel's modes) into out[ns], in a fixed order.
-// A block takes 2048 nodes or more; the partial sums of up to RED_HOST blocks
-// are added here, more of them on the device, where a second launch costs less
-// than the copy (40 cells of Nq = 5: 64 us for a norm, integrals, gather and
-// scatter with 512 blocks, 70 us with the second launch, 61 us so).
-constexpr int RED_HOST = 32;
+// A block takes 2048 nodes or more, but powers (mode 3), which are bound by the
+// power and not by memory, 256 (27 cells of Nq = 5, five FP64 states: 38 us with
+// 512 blocks, 59 us with 2048 nodes a block, 33 us so).  Up to RED_HOST partial
+// sums are added here, more of them on the device, where a second launch costs
+// less than the copy and the additions (integrals of one state, 73 blocks: 25.8
+// us here, 28.4 us there).
+constexpr int RED_HOST = 512;
 int reduce(rv_handle *h, const void *q, int mode, double *out, double pexp = 2.0)
 {
     if (!q)
         return fail(h, RV_E_ARG, "null state");
     const int ns = h->ns;
-    const int blocks =
-        (int)std::min<int64_t>(RED_BLOCKS, std::max<int64_t>(1, h->Np * h->K / 2048));
+    const int64_t n = h->Np * h->K;
+    const int blocks = (int)std::min<int64_t>(
+        RED_BLOCKS, std::max<int64_t>(1, mode == 3 ? (n + RED_THREADS - 1) / RED_THREADS : n / 2048));
+    const bool here = blocks * ns <= RED_HOST;
     auto run = [&](auto n) {
         constexpr int NS = decltype(n)::value;
         if (h->dtype == RV_F64)
@@ -1132,8 +1136,8 @@ int reduce(rv_handle *h, const void *q, int mode, double *out, double pexp = 2.0
     default: return fail(h, RV_E_UNSUPPORTED, "reduction over this number of states");
     }
     HIP_TRY(h, hipGetLastError());
-    double part[2 * RED_HOST * 5];
-    if (mode != 4 && blocks > RED_HOST) {
+    double part[2 * RED_HOST];
+    if (mode != 4 && !here) {
         double *sums = h->partials + (size_t)2 * RED_BLOCKS * ns;
         if (launch_slot_sums(h->partials, 2 * blocks, ns, 1, 2 * blocks, 0, 1, 1, sums,
                              h->stream) != 0) {
@@ -1147,8 +1151,8 @@ int reduce(rv_handle *h, const void *q, int mode, double *out, double pexp = 2.0
         std::copy(part, part + ns, out);
         return RV_OK;
     }
-    std::vector<double> many(blocks > RED_HOST ? (size_t)2 * blocks * ns : 0);
-    double *p = blocks > RED_HOST ? many.data() : part;
+    std::vector<double> many(here ? 0 : (size_t)2 * blocks * ns);
+    double *p = here ? part : many.data();
     HIP_TRY(h, hipMemcpyAsync(p, h->partials, (size_t)2 * blocks * ns * sizeof(double),
                               hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(h, hipStreamSynchronize(h->stream));
