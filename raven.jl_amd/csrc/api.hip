@@ -73,6 +73,7 @@ struct rv_handle {
     bool own_stream = false;
     int wpb = 1;      // waves per workgroup of a fused stage
     int wpb_rhs = 1;  // ... of a right-hand side alone (no q_out written)
+    bool wpb_set = false;  // by rv_set_waves_per_block
     StageLauncher launcher = nullptr;
     StageLauncher relax_launcher = nullptr;  // fused relaxation stage, when built
     // device buffers
@@ -782,19 +783,8 @@ int finish_setup(rv_handle *h, const double *D, const double *w)
         rk.relax = 1;
         h->relax_launcher = find_stage_launcher(rk);
     }
-    // waves per workgroup measured on MI355X for the 3-D column kernel on the
-    // 32^3 Nq = 8 Euler brick: a fused stage is fastest with four for FP64
-    // (0.50 ms against 0.52 ms with one or two) and two for FP32 (one, two
-    // and four within 2 %); a right-hand side alone with one for FP64
-    // (0.36 ms against 0.37 and 0.40 ms) and two for FP32
-    h->wpb = h->dim == 3 ? (h->dtype == RV_F32 ? 2 : 4) : 1;
-    h->wpb_rhs = h->dim == 3 && h->dtype == RV_F32 ? 2 : 1;
-    // grids of at most 1024 waves spread over the CUs (a workgroup of four
-    // waves each would leave half of them idle): 216 cells of Nq = 8 FP64
-    // 15.7 us per stage against 18.4, 343 of Nq = 7 16.8 against 21.4
-    const int epw = 64 / (nq * nq) < 1 ? 1 : 64 / (nq * nq);
-    if (h->dim == 3 && h->K <= (int64_t)1024 * epw)
-        h->wpb = h->wpb_rhs = 1;
+    h->wpb = default_waves(h->dim, nq, key.real_bytes, h->K, true);
+    h->wpb_rhs = default_waves(h->dim, nq, key.real_bytes, h->K, false);
     if (!h->launcher)
         return fail(h, RV_E_UNSUPPORTED,
                     "no kernel for dim=" + std::to_string(h->dim) + " nq=" + std::to_string(nq) +
@@ -1546,6 +1536,7 @@ int rv_set_waves_per_block(rv_handle *h, int waves_per_block)
         return fail(h, RV_E_ARG, "waves per block must be 1, 2 or 4");
     h->wpb = waves_per_block;
     h->wpb_rhs = waves_per_block;
+    h->wpb_set = true;
     return RV_OK;
 }
 
@@ -2896,14 +2887,21 @@ void batch_layout(rv_batch *b, std::vector<BatchItem> &items)
     b->nitems = (int64_t)items.size();
     if (b->tail_first < 0)
         b->tail_first = b->nitems;
-    // a kind launching on its own takes its first member's launch shape (the
-    // single operator's, autotuned or default)
+    // a kind launching on its own takes its first member's launch shape, if that
+    // was set or autotuned, or the default for the kind and all of its cells
     for (int p = 0; p < b->tail_mbegin; ++p) {
-        const int m = order[p];
-        if (p == 0 || kind[m] != kind[order[p - 1]])
-            b->kind_ranges.push_back({kind[m], b->slab_own[m], b->members[m]->wpb, p, p + 1});
+        if (p == 0 || kind[order[p]] != kind[order[p - 1]])
+            b->kind_ranges.push_back({kind[order[p]], b->slab_own[order[p]], 1, p, p + 1});
         else
             b->kind_ranges.back().mend = p + 1;
+    }
+    for (auto &r : b->kind_ranges) {
+        const rv_handle *h = b->members[order[r.mbegin]];
+        int64_t cells = 0;
+        for (int p = r.mbegin; p < r.mend; ++p)
+            cells += b->members[order[p]]->K;
+        r.wpb = kind_waves(b->dim, h->nq, h->law, h->dtype == RV_F64 ? 8 : 4, cells,
+                           h->wpb_set ? h->wpb : 0);
     }
 }
 

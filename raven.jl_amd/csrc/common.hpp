@@ -219,6 +219,36 @@ inline int64_t plane3_relax_slots(int nq, int law, int real_bytes, int geo, int6
     return (waves + wpb - 1) / wpb * wpb;
 }
 
+// Default waves per workgroup of a launch over K cells (rv_set_waves_per_block).
+// Measured on MI355X for the 3-D column kernel on 32^3 cells of Nq = 8: a fused
+// stage is fastest with four for FP64 (0.50 ms against 0.52 ms with one or two)
+// and two for FP32 (one, two and four within 2 %); a right-hand side alone with
+// one for FP64 (0.36 ms against 0.37 and 0.40 ms) and two for FP32.  Grids of at
+// most 1024 waves spread over the CUs (a workgroup of four waves each would leave
+// half of them idle): 216 cells of Nq = 8 FP64 15.7 us per stage against 18.4, 343
+// of Nq = 7 16.8 against 21.4.
+inline int default_waves(int dim, int nq, int real_bytes, int64_t K, bool write_q)
+{
+    const int epw = nq > 8 ? 1 : 64 / (nq * nq);
+    if (dim != 3 || K <= (int64_t)1024 * epw)
+        return 1;
+    return real_bytes == 4 ? 2 : write_q ? 4 : 1;
+}
+// ... and of a batch's launch of one kind, whose members have `cells` cells in all:
+// what the first member was given (chosen, 0: nothing), else one for FP64 Euler and
+// two for the others (the first member's own default would make the launch depend
+// on the members' order).  us per step, one / two / four waves: six members of 14^3
+// and one of 3^3 cells of Nq = 8 FP64 Euler 1473 / 1494 / 1548, Nq = 7 1205 / 1248 /
+// 1445, 4 of 32^3 of Nq = 7 8715 / 8993 / 10993; FP32 Euler 16 of 8^3 of Nq = 6 213 /
+// 204 / 203, advection 8 of 20^3 of Nq = 5 275 / 259 / 258; few cells: 3 of 8^3 of
+// Nq = 5 FP32 Euler 59 / 67 / 60.
+inline int kind_waves(int dim, int nq, int law, int real_bytes, int64_t cells, int chosen)
+{
+    if (chosen)
+        return chosen;
+    return law == LAW_EULER && real_bytes == 8 ? 1 : default_waves(dim, nq, 4, cells, true);
+}
+
 // Launch the fused stage for one kernel configuration; returns false when no
 // kernel is instantiated for it.
 using StageLauncher = int (*)(const StageParams &, void *stream, int waves_per_block);
