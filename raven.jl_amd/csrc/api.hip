@@ -1015,13 +1015,11 @@ int create_from_desc(const rv_desc *d, rv_handle *h)
 
 // whether a stage (write_q), or a right-hand side alone, streams dq and q_out
 // past L2 (which then keeps the q lines that face reads share)
-int16_t streams(const rv_handle *h, bool write_q)
+bool streams(const rv_handle *h, bool write_q)
 {
     const int b = h->dtype == RV_F32 ? 4 : 8;
     return launch_streams(h->dim, h->nq, h->law, b, h->geo, h->vflux, write_q,
-                          h->Np * h->ns * h->K * b)
-               ? 1
-               : 0;
+                          h->Np * h->ns * h->K * b);
 }
 
 StageParams stage_params(rv_handle *h)
@@ -1047,7 +1045,6 @@ StageParams stage_params(rv_handle *h)
     P.gamma = h->gamma;
     for (int c = 0; c < 3; ++c)
         P.u[c] = h->u[c];
-    P.streaming = streams(h, true);
     return P;
 }
 
@@ -1450,7 +1447,7 @@ int rv_get_info(const rv_handle *h, rv_info *info)
     info->geometry = h->geo == GEO_AFFINE ? RV_GEOM_AFFINE : RV_GEOM_GENERAL;
     info->faces_self = h->faces_self;
     info->faces_explicit = h->faces_explicit;
-    info->streaming = stage_params(const_cast<rv_handle *>(h)).streaming;
+    info->streaming = streams(h, true);
     info->ncells = h->K;
     const int64_t b = h->dtype == RV_F64 ? 8 : 4;
     const int64_t nodes = h->Np * h->K;

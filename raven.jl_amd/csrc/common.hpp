@@ -52,15 +52,18 @@ struct StageParams {
     void RV_GLOBAL *dq;          // register (R)
     double a;             // dq = a*dq + L
     double b_dt;          // q_out = q_in + b_dt*dq
-    int16_t read_dq;      // load dq (a != 0 or increment)
-    int16_t write_q;      // stage mode
-    int16_t dir_mask;     // active directions (bit d)
-    int16_t streaming;    // dq and q_out through L2 as streaming (non-temporal) accesses
+    // (fields of one word: batches read them through a table, where the scalar unit
+    // loads words and the vector unit anything shorter, for branches to wait for)
+    uint32_t read_dq : 1;    // load dq (a != 0 or increment)
+    uint32_t write_q : 1;    // stage mode
+    uint32_t streaming : 1;  // dq and q_out through L2 as streaming (non-temporal) accesses
+    uint32_t dir_mask : 8;   // active directions (bit d)
+    uint32_t unused : 21;
     // the launch's own shape (launch_stage): workgroups and waves in each.  The
     // kernels read it here, with the rest, and not through blockDim and gridDim,
     // which the runtime puts behind the arguments: two more lines to fetch
     uint32_t blocks;
-    int32_t wpb;
+    int32_t wpb, pad;
     const FaceRec RV_GLOBAL *faces;        // (2dim, K)
     const int64_t RV_GLOBAL *explicit_idx; // explicit face-node offsets
     // affine geometry: per cell, per direction: dRdX[d,d] (FP64)
