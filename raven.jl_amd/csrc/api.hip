@@ -688,29 +688,31 @@ __global__ void round_to_f32_kernel(const double *__restrict__ src, float *__res
         dst[i] = (float)src[i];
 }
 
-// The FP32 copies of the general geometry (and MJ) that the 2-D and 3-D stage
-// kernels of an FP32 handle read (StageParams::vgeo32 ...), made again after every
-// change of the FP64 arrays.
+// The FP32 copies of the general geometry that the 2-D and 3-D stage kernels of
+// an FP32 handle read (StageParams::vgeo32 ...), and of MJ for the 3-D column
+// kernel's relaxation stage, made again after every change of the FP64 arrays.
 int refresh_geo32(rv_handle *h)
 {
     if (!(h->dtype == RV_F32 && h->geo == GEO_GENERAL && h->dim >= 2) || h->K <= 0)
         return RV_OK;
     const int64_t nv = h->K * h->dim * h->dim * h->Np, nm = h->K * h->Np,
                   ns = h->K * 2 * h->dim * (h->dim + 1) * h->nfp;
+    const bool mj = h->dim == 3 && h->vflux == 0;
     int rc;
     if (!h->vgeo32 && ((rc = dalloc(h, &h->vgeo32, nv)) || (rc = dalloc(h, &h->mji32, nm)) ||
-                       (rc = dalloc(h, &h->sgeo32, ns)) || (rc = dalloc(h, &h->mj32, nm))))
+                       (rc = dalloc(h, &h->sgeo32, ns)) || (mj && (rc = dalloc(h, &h->mj32, nm)))))
         return rc;
     const struct {
         const double *src;
         float *dst;
         int64_t n;
     } parts[] = {{h->vgeo, h->vgeo32, nv}, {h->mji, h->mji32, nm}, {h->sgeo, h->sgeo32, ns},
-                 {h->MJ, h->mj32, nm}};
+                 {h->MJ, h->mj32, mj ? nm : 0}};
     for (const auto &c : parts)
-        hipLaunchKernelGGL(round_to_f32_kernel,
-                           dim3((unsigned)std::min<int64_t>((c.n + 255) / 256, 4096)), dim3(256),
-                           0, h->stream, c.src, c.dst, c.n);
+        if (c.n > 0)
+            hipLaunchKernelGGL(round_to_f32_kernel,
+                               dim3((unsigned)std::min<int64_t>((c.n + 255) / 256, 4096)),
+                               dim3(256), 0, h->stream, c.src, c.dst, c.n);
     HIP_TRY(h, hipGetLastError());
     return RV_OK;
 }
@@ -1592,7 +1594,6 @@ int rv_enable_mortars(rv_handle *h, const int32_t *face_kind, const int64_t *par
             for (int t = 0; t < 4; ++t)
                 pr.part[t] = partner[4 * (e * nf + f) + t];
             pr.f = f;
-            pr.kind = k;
             (k == 2 ? pairs : hanging).push_back(pr);
         }
     }

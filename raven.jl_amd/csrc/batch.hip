@@ -8,7 +8,7 @@
 // running at the same time mostly execute the same code.  Each persistent wave
 // walks the list with a stride of the launched wave count and hands every item
 // to the same per-wave routine the single-operator kernels use
-// (stage_wave / plane3_wave), with that member's StageParams read from a
+// (quad2_group / plane3_wave), with that member's StageParams read from a
 // device table.  Members are restricted to affine geometry and the Rusanov
 // flux (the brick solves batched and served here); 2-D members take Nq 2..8,
 // 3-D members Nq 4..8.  2-D items run the node kernel's group routine

@@ -79,8 +79,8 @@ struct StageParams {
     const double RV_GLOBAL *mji;   // (K, Np)
     const double RV_GLOBAL *mj;    // (K, Np) = wJ
     const double RV_GLOBAL *sgeo;  // (K, 2dim, dim+1, Nfp): n_c ..., wsJ
-    // FP32 handles, 2-D and 3-D general cells: vgeo, mji, sgeo and mj rounded to
-    // FP32 once (the stage kernels round every use of them to the state type,
+    // FP32 handles, 2-D and 3-D general cells: vgeo, mji, sgeo and (for the 3-D column
+    // kernel) mj rounded to FP32 once (the stage kernels round every use of them to the state type,
     // so reading these gives the same results with half the geometry bytes)
     const float RV_GLOBAL *vgeo32;
     const float RV_GLOBAL *mji32;
@@ -264,12 +264,12 @@ struct KernelKey {
 
 // Mortar coupling of hanging faces (mortar.hip), launched after a stage.
 // One non-conforming face of a mortar cell: its cell e (and slot li in the
-// list of mortar cells), face f, kind (1 hanging, 2 covered) and partners
-// (hanging: coarse cell, sub-face; covered: the 2^(dim-1) fine cells)
+// list of mortar cells), face f and partners (hanging: coarse cell, sub-face;
+// covered: the 2^(dim-1) fine cells; covered faces come first)
 struct MortarPair {
     int64_t e, li;
     int64_t part[4];
-    int32_t f, kind;
+    int64_t f;
 };
 
 struct MortarParams {

@@ -185,8 +185,7 @@ __device__ __forceinline__ double log_factor(double a, double b, double s, doubl
 
 // A node of a line, what the two-point flux takes from it, and the flux of a
 // pair along a metric vector m (GEN) or along component 0 of the (permuted)
-// velocity.  LDS holds NC values per node: lds_values(q) writes the first
-// 2 + DIM (1 for advection).
+// velocity.  LDS holds the NV values of a node that values() forms.
 template <int DIM, int LAW, int VF, typename R, bool GEN>
 struct TwoPoint {
     static constexpr int NS = LawInfo<DIM, LAW>::NS;
@@ -365,7 +364,7 @@ struct FD {
     static constexpr int CS = NL * PR;
     static constexpr int CMP = C * CS;  // one component of the workgroup's cells
     // components: rho, b, then u, v, w and (affine) u, v again
-    static constexpr int NC = TP::NV + (GEN || TP::ADV ? 0 : DIM - 1);
+    static constexpr int NC = TP::NV + (GEN ? 0 : DIM - 1);
     static constexpr int POOL = CMP * (NC > NS ? NC : NS);
     // FP64: the line's sums take 2 Nq Ns registers; partners are read from LDS
     // at every pair instead of being held, so that three waves share a SIMD
@@ -414,7 +413,8 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
     using TP = typename T::TP;
     using Node = typename TP::Node;
     constexpr int NS = T::NS, NP = T::NP, NL = T::NL, NF = T::NF, PR = T::PR, CMP = T::CMP;
-    constexpr bool GEN = T::GEN, ADV = TP::ADV;
+    constexpr bool GEN = T::GEN;
+    static_assert(TP::EC && DIM > 1, "the line kernel's forms (fd_has_line_kernel)");
     __shared__ __align__(16) R lds[T::POOL];
     const int t = threadIdx.x;
     const int64_t cell0 = xcd_remap(blockIdx.x, P.blocks) * T::C;
@@ -451,7 +451,7 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
 #pragma unroll
                 for (int k = 0; k < TP::NV; ++k)
                     x[k * CMP] = val[k];
-                if constexpr (!GEN && !ADV) {
+                if constexpr (!GEN) {
 #pragma unroll
                     for (int d = 0; d + 1 < DIM; ++d)
                         x[(TP::NV + d) * CMP] = val[2 + d];
@@ -496,30 +496,19 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
         const Line line = line_of(t);
         int lbase = line.lbase;
         const int64_t e = cell(line.c);
-        // the law as the line sees it: its direction first (affine cells)
-        Law<DIM, LAW, R> lawp = law;
-        if constexpr (ADV && !GEN && DIM > 1) {
-#pragma unroll
-            for (int d = 0; d < DIM; ++d)
-                lawp.u[d] = dir == 0   ? law.u[d]
-                            : dir == 1 ? law.u[(d + 1) % DIM]
-                                       : law.u[(d + 2) % DIM];
-        }
         auto load = [&](int n) {
             const R *x = lds + lbase + n * lstr;
             R val[TP::NV];
             val[0] = x[0];
-            if constexpr (!ADV) {
-                val[1] = x[CMP];
+            val[1] = x[CMP];
 #pragma unroll
-                for (int d = 0; d < DIM; ++d)
-                    val[2 + d] = x[uoff + (2 + d) * CMP];
-            }
+            for (int d = 0; d < DIM; ++d)
+                val[2 + d] = x[uoff + (2 + d) * CMP];
             return TP::node(law, val);
         };
         // FP32 state reads the FP32 copies of the geometry (every use
         // rounds to the state's type)
-        constexpr bool G32 = GEN && DIM > 1 && sizeof(R) == 4;
+        constexpr bool G32 = GEN && sizeof(R) == 4;
         using GT = typename std::conditional<G32, float, double>::type;
         const GT RV_GLOBAL *vgeo, *sgeo;
         if constexpr (G32)
@@ -555,7 +544,7 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
 #pragma unroll
             for (int s = 0; s < NS; ++s)
                 comp[s] = s;
-            if constexpr (!GEN && !ADV && DIM > 1) {
+            if constexpr (!GEN) {
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) {
                     const int k = dir + d;
@@ -598,38 +587,36 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
         // compared without squares, which would leave the type's range, and
         // each is kept where the flux's reciprocals are normal numbers (FP64
         // takes one of the product of the sums of rho and of b).
-        int rough = 0;  // 0: short series, 1: long series, 2: logarithms
-        if constexpr (TP::EC) {
-            constexpr int W = sizeof(R) / 4;  // 32-bit words per value
-            constexpr R LEAST = W == 2 ? R(1e-140) : R(1e-37), MOST = W == 2 ? R(1e140) : R(1e37);
-            const uint32_t *w = reinterpret_cast<const uint32_t *>(lds) + W * lbase + (W - 1);
-            bool ok[2] = {true, true};
+        constexpr int W = sizeof(R) / 4;  // 32-bit words per value
+        constexpr R LEAST = W == 2 ? R(1e-140) : R(1e-37), MOST = W == 2 ? R(1e140) : R(1e37);
+        const uint32_t *w = reinterpret_cast<const uint32_t *>(lds) + W * lbase + (W - 1);
+        bool ok[2] = {true, true};
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                uint32_t lo = w[W * k * CMP], hi = lo;
+        for (int k = 0; k < 2; ++k) {
+            uint32_t lo = w[W * k * CMP], hi = lo;
 #pragma unroll
-                for (int n = 1; n < NQ; ++n) {
-                    const uint32_t v = w[W * (n * lstr + k * CMP)];
-                    lo = v < lo ? v : lo;
-                    hi = v > hi ? v : hi;
-                }
-                R x0, x1;
-                if constexpr (W == 2) {
-                    x0 = __longlong_as_double((long long)((uint64_t)lo << 32));
-                    x1 = __longlong_as_double((long long)((uint64_t)hi << 32 | 0xffffffffu));
-                } else {
-                    x0 = __uint_as_float(lo);
-                    x1 = __uint_as_float(hi);
-                }
-                const R d = fabs(x1 - x0), s = x1 + x0;
-                ok[0] = ok[0] && x0 > LEAST && x1 < MOST;
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    ok[j] = ok[j] && d < R(LogSeries<R>::FLIMIT[j]) * s;
+            for (int n = 1; n < NQ; ++n) {
+                const uint32_t v = w[W * (n * lstr + k * CMP)];
+                lo = v < lo ? v : lo;
+                hi = v > hi ? v : hi;
             }
-            ok[1] = ok[1] && ok[0];
-            rough = __all(ok[1]) ? 0 : __all(ok[0]) ? 1 : 2;
+            R x0, x1;
+            if constexpr (W == 2) {
+                x0 = __longlong_as_double((long long)((uint64_t)lo << 32));
+                x1 = __longlong_as_double((long long)((uint64_t)hi << 32 | 0xffffffffu));
+            } else {
+                x0 = __uint_as_float(lo);
+                x1 = __uint_as_float(hi);
+            }
+            const R d = fabs(x1 - x0), s = x1 + x0;
+            ok[0] = ok[0] && x0 > LEAST && x1 < MOST;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                ok[j] = ok[j] && d < R(LogSeries<R>::FLIMIT[j]) * s;
         }
+        ok[1] = ok[1] && ok[0];
+        // 0: short series, 1: long series, 2: logarithms
+        const int rough = __all(ok[1]) ? 0 : __all(ok[0]) ? 1 : 2;
         auto pairs = [&](auto series) {
             constexpr int SERIES = decltype(series)::value;
 #pragma unroll
@@ -660,9 +647,9 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
 #pragma unroll
                         for (int d = 0; d < DIM; ++d)
                             m[d] = Dni * lb[d] - Din * la[d];
-                        TP::template flux<SERIES>(lawp, a, b, m, F);
+                        TP::template flux<SERIES>(law, a, b, m, F);
                     } else {
-                        TP::template flux<SERIES>(lawp, a, b, nullptr, F);
+                        TP::template flux<SERIES>(law, a, b, nullptr, F);
                         wi = S_in[i * NQ + n], wn = S_in[n * NQ + i];
                     }
 #pragma unroll
@@ -675,9 +662,9 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
         };
         if (rough == 0) {
             pairs(std::integral_constant<int, 1>{});
-        } else if (TP::EC && rough == 1) {
+        } else if (rough == 1) {
             pairs(std::integral_constant<int, 0>{});
-        } else if constexpr (TP::EC) {
+        } else {
             // a rolled loop (its indexes are the same on every lane): the
             // accumulators are addressed by weights that are zero elsewhere,
             // by the partner's only where registers allow the outer loop to
@@ -707,10 +694,10 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
 #pragma unroll
                         for (int d = 0; d < DIM; ++d)
                             m[d] = Dni * lb[d] - Din * la[d];
-                        TP::template flux<-1>(lawp, a, b, m, F);
+                        TP::template flux<-1>(law, a, b, m, F);
                         wi = R(1), wn = R(-1);
                     } else {
-                        TP::template flux<-1>(lawp, a, b, nullptr, F);
+                        TP::template flux<-1>(law, a, b, nullptr, F);
                         wi = S_in[i * NQ + n], wn = S_in[n * NQ + i];
                     }
 #pragma unroll
@@ -747,17 +734,17 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
                 // twopointflux(q-, q+)' n; on an affine face n = +-e_dir
                 static_assert(SF == VF, "the surface flux is Rusanov or the volume form's own");
                 R val[TP::NV], F[NS];
-                TP::values(lawp, qp[side], val);
-                TP::template flux<-1>(lawp, load(end), TP::node(lawp, val), nv, F);
+                TP::values(law, qp[side], val);
+                TP::template flux<-1>(law, load(end), TP::node(law, val), nv, F);
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
                     nf[s] = GEN || side ? F[s] : -F[s];
             } else if constexpr (GEN) {
-                S::nflux_general(lawp, nv, qm[side], qp[side], nf);
+                S::nflux_general(law, nv, qm[side], qp[side], nf);
             } else {
                 R fm[NS];
-                lawp.flux_row(0, qm[side], fm);
-                S::nflux_axis(lawp, 0, side ? R(1) : R(-1), fm, qm[side], qp[side], nf);
+                law.flux_row(0, qm[side], fm);
+                S::nflux_axis(law, 0, side ? R(1) : R(-1), fm, qm[side], qp[side], nf);
             }
 #pragma unroll
             for (int s = 0; s < NS; ++s)
@@ -810,7 +797,7 @@ __device__ __forceinline__ void fd_stage(const StageParams &P)
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 int k = s;
-                if constexpr (!GEN && !ADV && DIM > 1) {
+                if constexpr (!GEN) {
                     if (s > 0 && s <= DIM)
                         k = 1 + (s - 1 + d) % DIM;
                 }

@@ -14,8 +14,9 @@
 // the transpose of the interpolation, so the fluxes through the two sides of
 // the mortar cancel exactly up to rounding (discrete conservation).  The stage
 // kernel leaves these faces out (their lift weight is zero on the device).
-//  * mortar_face_kernel, one wave per sub-face of a (cell, face) pair, runs before the stage kernel on the same stream: the face's lift L at
-//    its face nodes (the update is delta = -MJI L), into a per-face buffer
+//  * mortar_face_kernel, one wave per sub-face of a (cell, face) pair, runs
+//    before the stage kernel on the same stream: the face's lift L at its face
+//    nodes (the update is delta = -MJI L), into a per-face buffer
 //    (the faces only read q_in, so they are independent of each other and of
 //    the stage): L = wsJ_f nf_s on the fine side, minus the projection on the
 //    coarse side;
@@ -56,8 +57,8 @@ __global__ void __launch_bounds__(64 << (DIM - 1)) mortar_face_kernel(const Mort
     __shared__ R pass1[NSUB][NS][NFP];
     const StageParams &P = M.stage;
     const Law<DIM, LAW, R> law(P);
-    // the wave's non-conforming (cell, face) pair: its cell, face, kind and
-    // partners in one record (a wave past the last hanging face has none)
+    // the wave's non-conforming (cell, face) pair: its cell, face and partners in
+    // one record (a wave past the last hanging face has none)
     const int w = (int)wave_uniform(threadIdx.x >> 6), m = threadIdx.x & 63;
     const bool covered = blockIdx.x < M.ncovered;
     const int64_t ip = covered ? blockIdx.x
@@ -66,7 +67,7 @@ __global__ void __launch_bounds__(64 << (DIM - 1)) mortar_face_kernel(const Mort
     asm volatile("" ::"s"(M.sgeo), "s"(M.halves), "s"(M.delta), "s"(P.q_in));
     const MortarPair &pr = M.pairs[ip < M.npairs ? ip : M.npairs - 1];
     const int64_t e = pr.e, li = pr.li, p0 = pr.part[0], p1 = pr.part[1], pw = pr.part[w];
-    const int f = pr.f;
+    const int f = (int)pr.f;
     asm volatile("" ::"s"(e), "s"(li), "s"(p0), "s"(p1), "s"(pw), "s"(f));
     const bool on = m < NFP && ip < M.npairs;
     const int a = m % NQ, b = m / NQ;  // face node m = a + NQ*b (b = 0 in 2-D)

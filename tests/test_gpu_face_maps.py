@@ -88,3 +88,24 @@ def test_rhs(torch, R, dim, nq, geometry, form, face, line, dtype):
     err = rel_l2(dq.double().cpu().numpy().reshape(-1), want)
     print(f"   dq {err:.2e}", flush=True)
     assert err <= (1e-12 if dtype == "f64" else 1e-4)
+
+
+@pytest.mark.parametrize("dim,nq,form", [(2, 4, "weak"), (2, 4, "ec"), (3, 3, "ec"), (3, 3, "weak")])
+def test_fp32_geometry_copies(torch, R, dim, nq, form):
+    """An FP32 handle of curved cells holds, beyond the FP64 handle's arrays, the
+    copies its stages read: metric terms, 1 / MJ and faces, and MJ where the
+    weak form's 3-D relaxation stage reads it."""
+    n = [3, 2, 2][:dim]
+    grid = R.generate(R.GridManager(R.LobattoCell(*([nq] * dim)), R.brick(
+        [PB.julia_range(0, 1, k + 1) for k in n], (False,) * dim)), warp={2: warp2, 3: warp3}[dim])
+    vol = R.WeakForm() if form == "weak" else R.FluxDifferencingForm(R.EntropyConservativeFlux())
+    held = []
+    for dtype in ("f32", "f64"):
+        dg = R.DGSEM(law=R.EulerLaw(dim), grid=grid, dtype=dtype, volume_form=vol,
+                     surface_numericalflux=R.RusanovFlux())
+        held.append(dg.info.device_bytes)
+    copies = dg.K * (dg.Np * (dim * dim + 1) + 2 * dim * (dim + 1) * nq ** (dim - 1))
+    if form == "weak" and dim == 3:
+        copies += dg.K * dg.Np
+    tables = 0 if form == "weak" else 2 * nq * nq  # pair weights, in the state's type
+    assert held[0] - held[1] == 4 * (copies - tables)
