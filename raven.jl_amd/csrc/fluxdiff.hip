@@ -33,9 +33,9 @@
 //
 // It is bound by FP64 (or unpacked FP32) vector issue and HBM together: 52 or
 // 60 instructions a pair (short or long series), 10.5 pairs a node at Nq = 8.
-// On 32^3 cells of Nq = 8 a stage takes 0.80 ms in FP64 (a thread per node
-// with the pairs' terms exchanged through an LDS buffer took 2.00 ms):
-// 2.95 GB moved (3.7 TB/s), vector units busy 61 % of the cycles.
+// On 32^3 cells of Nq = 8 a FP64 stage takes 0.86 ms (a thread per node with the
+// pairs' terms exchanged through an LDS buffer took 2.00 ms): 2.94 GB moved (3.4
+// TB/s), vector units busy 66 % of the cycles.
 //
 // The node kernel (fd_stage_node; everything else): a lane per node, each pair
 // evaluated from both ends.  The fluxes of the central forms cost little, and
