@@ -350,10 +350,20 @@ int launch_quad2(const StageParams &P, void *stream, int wpb)
     constexpr int G = quad2_group_waves<NQ>();
     // (curved cells: one node per lane, whose metric terms are bytes enough in
     // flight: 2 took 44 to 51 us against 41 to 46 us per FP64 Euler stage of
-    // 1.4 to 1.6 M nodes, advection likewise)
+    // 1.4 to 1.6 M nodes, advection likewise; one exception below)
     constexpr int V = GEO == GEO_GENERAL ? 1 : quad2_nodes_per_lane<LAW, R>();
     if (P.K <= 0)
         return 0;
+    // Curved FP64 advection whose cells fill a wave (Nq = 8), right-hand side
+    // alone: no q_out and dq_old to move, so one node per lane has too few bytes
+    // in flight.  us with 1 / 2 nodes: 125^2 cells 13.4 / 13.5, 177^2 23.9 /
+    // 22.7, 250^2 56.3 / 49.3, 433^2 193 / 174; smaller cells share waves and
+    // lose up to 12 % (Nq = 6, 167^2: 12.0 / 13.5).
+    if constexpr (LAW == LAW_ADVECTION && GEO == GEO_GENERAL && NQ * NQ == 64 &&
+                  sizeof(R) == 8) {
+        if (!P.write_q && P.K > 20000)
+            return launch_quad2_v<NQ, LAW, R, FLUX, GEO, 2>(P, stream, wpb);
+    }
     // A grid that leaves the device room for its waves is not bound by bytes
     // but by one wave's pass through the code, fetched cold at each launch, and
     // V nodes per lane make that V times as long: one node per lane up to 24
